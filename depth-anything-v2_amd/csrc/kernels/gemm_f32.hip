@@ -1,18 +1,19 @@
 // fp32 and fp16 paths of the precision modes (DAV2_CREATE_FORCE_FP32 /
 // FORCE_FP16): the linear and convolution GEMMs in float32 on the MFMA
-// (v_mfma_f32_16x16x4_f32), with the epilogues of the int8 GEMM, and the
-// fp32 im2col that feeds convolutions.
+// (v_mfma_f32_16x16x4_f32; v_mfma_f32_16x16x32_f16 on operands rounded to
+// binary16), with the epilogues of the int8 GEMM, and the fp32 im2col that
+// feeds convolutions.
 //
 // fp16 arithmetic comes in the reference's two forms. Cooperative-matrix
 // linears (linear_coop_fp16.glsl via linear_fp16* with cooperative_matrix_fp16,
 // src/operators.cpp:540-768): operands rounded to binary16, exact products,
-// fp32 accumulation. The fp32 GEMM does this with half_operands: both tiles
-// are rounded to binary16 as they are staged, and the product of two binary16
-// values is exact in fp32. Native binary16 shaders (prepare_tokens_fp16,
-// project_tokens_fp16, conv_transpose_nonoverlap_fp16): every product is a
-// binary16 multiplication, widened and added to an fp32 sum in k order;
-// gemm_h16p_kernel does exactly that on the VALU, so its results match the
-// oracle bit for bit.
+// fp32 accumulation. The fp32 GEMM does this with half_operands: both operands
+// are rounded to binary16 on their way from LDS to v_mfma_f32_16x16x32_f16,
+// whose products are exact and whose sums are fp32. Native binary16 shaders
+// (prepare_tokens_fp16, project_tokens_fp16, conv_transpose_nonoverlap_fp16):
+// every product is a binary16 multiplication, widened and added to an fp32 sum
+// in k order; gemm_h16p_kernel does exactly that on the VALU, so its results
+// match the oracle bit for bit.
 //
 // Reference: linear_tiled.glsl / linear_vec*.glsl (src/operators.cpp:882-955),
 // conv2d (:1528-1676), conv_transpose_nonoverlap (:1807-1861),
@@ -20,12 +21,16 @@
 // each dot product in its own tile order; fp32 results are compared within a
 // tolerance, not bit for bit.
 //
-// Tiles: 64x64 outputs per 256-thread workgroup, 2x2 waves of 32x32; K in
-// steps of 32 floats through a two-stage LDS ring filled from registers
-// (the next step's loads are in flight while the current one multiplies).
-// A lane's 16-byte fragment holds 4 consecutive k of its row; the 4 MFMAs of
-// a fragment take element e of every lane, so each MFMA sums k = 4g + e over
-// the lane groups g and the four together cover 16 k.
+// K advances in stages of 32 floats copied straight from global memory into an
+// LDS ring (global_load_lds_dwordx4), XOR-swizzled 128-byte rows as in the int8
+// GEMM, one barrier per stage; the operands of the next 16 k are read from LDS
+// while the present ones multiply. A lane's 16-byte fragment holds 4
+// consecutive k of its row; the 4 MFMAs of a fragment take element e of every
+// lane, so each MFMA sums k = 4g + e over the lane groups g and the four
+// together cover 16 k. What bounds it: the fp32 MFMA (157 TFLOP/s), of which
+// a chip full of tiles reaches 110 (the same loop without the copies: 135).
+
+#include <type_traits>
 
 #include "common.h"
 #include "dav2_hip.h"
@@ -34,8 +39,8 @@ namespace {
 
 using namespace dav2k;
 
-constexpr int kBM = 64, kBN = 64, kBK = 32;  // tile rows, tile columns, floats per K step
-constexpr int kLdsRow = kBK + 4;             // padded LDS row (floats)
+constexpr int kBM = 64, kBN = 64;  // gemm_h16p_kernel's tile
+constexpr int kBK = 32;            // floats per K step
 
 struct F32Params {
     const float* a;
@@ -50,132 +55,237 @@ struct F32Params {
     const float* gamma;
     uint32_t relu_output;
     uint32_t convt_k, convt_w, convt_h, convt_c;
-    uint32_t half_operands;  // round both operands to binary16 when staged
+    uint32_t half_operands;  // round both operands to binary16
 };
 
+// Four consecutive weight rows n .. n + 3 of activation row m. Row-major
+// epilogues write them as one float4 when `vec` (n % 4 == 0 rows and 16-byte
+// aligned buffers); the channel-major ones run along m across the lanes.
 template <int EPI>
-DAV2_DEV void store_f32(const F32Params& g, uint32_t m, uint32_t n, float acc) {
-    if (EPI == DAV2_GEMM_EPI_CONVT) {
-        const uint32_t kidx = n / g.convt_c, oc = n - kidx * g.convt_c;
-        const float v = acc + (g.bias ? g.bias[oc] : 0.0f);
-        const uint32_t k = g.convt_k;
-        const uint32_t iy = m / g.convt_w, ix = m - iy * g.convt_w;
-        const uint32_t ky = kidx / k, kx = kidx - ky * k;
-        const uint32_t ow = g.convt_w * k, oh = g.convt_h * k;
-        g.out[(static_cast<uint64_t>(oc) * oh + iy * k + ky) * ow + ix * k + kx] = v;
-        return;
-    }
-    const float v = acc + (g.bias ? g.bias[n] : 0.0f);
-    if (EPI == DAV2_GEMM_EPI_TRANSPOSED) {
-        const uint64_t idx = static_cast<uint64_t>(n) * g.out_row_stride + m + g.out_row_offset;
-        float o = v;
-        if (g.residual) o = o + g.residual[idx];
-        if (g.relu_output) o = fmaxf(o, 0.0f);
-        g.out[idx] = o;
+DAV2_DEV void store_f32(const F32Params& g, uint32_t m, uint32_t n, const float (&acc)[4], bool vec) {
+    if (EPI == DAV2_GEMM_EPI_CONVT || EPI == DAV2_GEMM_EPI_TRANSPOSED) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (n + r >= g.n) return;
+            if (EPI == DAV2_GEMM_EPI_CONVT) {
+                const uint32_t kidx = (n + r) / g.convt_c, oc = (n + r) - kidx * g.convt_c;
+                const float v = acc[r] + (g.bias ? g.bias[oc] : 0.0f);
+                const uint32_t k = g.convt_k;
+                const uint32_t iy = m / g.convt_w, ix = m - iy * g.convt_w;
+                const uint32_t ky = kidx / k, kx = kidx - ky * k;
+                const uint32_t ow = g.convt_w * k, oh = g.convt_h * k;
+                g.out[(static_cast<uint64_t>(oc) * oh + iy * k + ky) * ow + ix * k + kx] = v;
+            } else {
+                const uint64_t idx = static_cast<uint64_t>(n + r) * g.out_row_stride + m + g.out_row_offset;
+                float o = acc[r] + (g.bias ? g.bias[n + r] : 0.0f);
+                if (g.residual) o = o + g.residual[idx];
+                if (g.relu_output) o = fmaxf(o, 0.0f);
+                g.out[idx] = o;
+            }
+        }
         return;
     }
     const uint64_t idx = (static_cast<uint64_t>(m) + g.out_row_offset) * g.n + n;
-    if (EPI == DAV2_GEMM_EPI_ROW_GELU) {
-        g.out[idx] = gelu_erfcc(v);
-    } else if (EPI == DAV2_GEMM_EPI_ROW_LAYERSCALE) {
-        const float scaled = v * g.gamma[n];  // add_scaled.glsl:26-30, no contraction
-        g.out[idx] = g.residual[idx] + scaled;
+    float v[4], res[4], gam[4];
+    if (vec) {
+        const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 b = g.bias ? *reinterpret_cast<const float4*>(g.bias + n) : zero;
+        v[0] = acc[0] + b.x, v[1] = acc[1] + b.y, v[2] = acc[2] + b.z, v[3] = acc[3] + b.w;
+        if (EPI == DAV2_GEMM_EPI_ROW_LAYERSCALE) {
+            const float4 s = *reinterpret_cast<const float4*>(g.gamma + n);
+            const float4 x = *reinterpret_cast<const float4*>(g.residual + idx);
+            gam[0] = s.x, gam[1] = s.y, gam[2] = s.z, gam[3] = s.w;
+            res[0] = x.x, res[1] = x.y, res[2] = x.z, res[3] = x.w;
+        }
     } else {
-        g.out[idx] = v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bool in = n + r < g.n;
+            v[r] = acc[r] + (g.bias && in ? g.bias[n + r] : 0.0f);
+            if (EPI == DAV2_GEMM_EPI_ROW_LAYERSCALE) {
+                gam[r] = in ? g.gamma[n + r] : 0.0f;
+                res[r] = in ? g.residual[idx + r] : 0.0f;
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (EPI == DAV2_GEMM_EPI_ROW_GELU) v[r] = gelu_erfcc(v[r]);
+        if (EPI == DAV2_GEMM_EPI_ROW_LAYERSCALE) {
+            const float scaled = v[r] * gam[r];  // add_scaled.glsl:26-30, no contraction
+            v[r] = res[r] + scaled;
+        }
+    }
+    if (vec) {
+        *reinterpret_cast<float4*>(g.out + idx) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (n + r < g.n) g.out[idx + r] = v[r];
     }
 }
 
 template <int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(F32Params g) {
-    __shared__ __attribute__((aligned(16))) float as[2][kBM * kLdsRow];
-    __shared__ __attribute__((aligned(16))) float bs[2][kBN * kLdsRow];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const uint32_t row0 = blockIdx.x * kBM, col0 = blockIdx.y * kBN;
+DAV2_DEV bool vector_rows(const F32Params& g) {
+    if (EPI == DAV2_GEMM_EPI_CONVT || EPI == DAV2_GEMM_EPI_TRANSPOSED) return false;
+    const uintptr_t any = reinterpret_cast<uintptr_t>(g.out) | reinterpret_cast<uintptr_t>(g.bias) |
+                          reinterpret_cast<uintptr_t>(g.gamma) | reinterpret_cast<uintptr_t>(g.residual);
+    return g.n % 4u == 0 && (any & 15u) == 0;
+}
+
+// BN weight rows (operand P of the MFMA, whose four result registers are then
+// consecutive output columns) x BM activation rows per workgroup, WN x WM
+// waves.
+template <int BN, int BM, int WN, int WM, int STAGES, bool HALF, int EPI>
+__global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
+    constexpr int NW = WN * WM, TN = BN / WN / 16, TM = BM / WM / 16;
+    constexpr int COPIES = (BN + BM) / 8;  // 1 KiB global -> LDS copies (8 rows of 128 bytes) per stage
+    constexpr int LPW = (COPIES + NW - 1) / NW;
+    constexpr int STAGE_BYTES = (BN + BM) * 128;
+    static_assert(TN * WN * 16 == BN && TM * WM * 16 == BM, "whole MFMA blocks per wave");
+    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave / WM, wm = wave % WM;
+    uint32_t tm, tn;
+    tile_of(tm, tn);
+    const uint32_t row0 = tm * BM, col0 = tn * BN;
     const int steps = static_cast<int>((g.k + kBK - 1) / kBK);
 
-    // Thread t moves float4 t and t + 256 of each 64 x 32 operand tile:
-    // tile row idx / 8, floats 4 (idx % 8) .. +3. Rows past the matrix and
-    // k past K read zeros (K is a multiple of 4, so a float4 is all in or out).
-    float4 ra[2], rb[2];
-    auto fetch = [&](uint32_t k0) {
+    // Copy c brings stage rows 8 c .. + 7, lane l row + l / 8 and the 16-byte
+    // chunk that swz maps to l % 8; wave w takes copies i NW + w (past the
+    // last one it repeats that one, the same bytes). Rows past the
+    // matrix read its last row (never stored), chunks past K chunk 0 of the
+    // row (masked below).
+    const float* src[LPW];
+    uint32_t chunk_k[LPW];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = tid + 256 * i;
-            const uint32_t r = static_cast<uint32_t>(idx >> 3), kk = k0 + 4u * (idx & 7);
-            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-            ra[i] = row0 + r < g.m && kk < g.k
-                        ? *reinterpret_cast<const float4*>(g.a + static_cast<uint64_t>(row0 + r) * g.lda + kk)
-                        : zero;
-            rb[i] = col0 + r < g.n && kk < g.k
-                        ? *reinterpret_cast<const float4*>(g.b + static_cast<uint64_t>(col0 + r) * g.ldb + kk)
-                        : zero;
-        }
-    };
-    auto stash = [&](int s) {
+    for (int i = 0; i < LPW; ++i) {
+        const uint32_t srow = 8u * min(i * NW + wave, COPIES - 1) + (lane >> 3);
+        chunk_k[i] = 4u * ((lane & 7) ^ ((srow >> 1) & 7u));
+        src[i] = srow < static_cast<uint32_t>(BN)  // uniform per instruction (BN % 8 == 0)
+                     ? g.b + min(col0 + srow, g.n - 1) * g.ldb
+                     : g.a + min(row0 + srow - BN, g.m - 1) * g.lda;
+    }
+    auto issue = [&](int step) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = tid + 256 * i;
-            const int off = (idx >> 3) * kLdsRow + 4 * (idx & 7);
-            float4 va = ra[i], vb = rb[i];
-            if (g.half_operands) {
-                va = make_float4(round_half(va.x), round_half(va.y), round_half(va.z), round_half(va.w));
-                vb = make_float4(round_half(vb.x), round_half(vb.y), round_half(vb.z), round_half(vb.w));
-            }
-            *reinterpret_cast<float4*>(&as[s][off]) = va;
-            *reinterpret_cast<float4*>(&bs[s][off]) = vb;
+        for (int i = 0; i < LPW; ++i) {
+            const uint32_t kk = static_cast<uint32_t>(step) * kBK + chunk_k[i];
+            copy16_to_lds(src[i] + (kk < g.k ? kk : 0u),
+                          smem + (step % STAGES) * STAGE_BYTES + min(i * NW + wave, COPIES - 1) * 1024);
         }
     };
 
-    v4f acc[2][2];
+    v4f acc[TN][TM];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    const int frag = (lane & 15) * kLdsRow + 4 * (lane >> 4);
-    for (int step = 0; step < steps; ++step) {
-        const int s = step & 1;
-        if (step + 1 < steps) fetch(static_cast<uint32_t>(step + 1) * kBK);
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float4 fa[2], fb[2];
+    for (int s = 0; s < STAGES; ++s)
+        if (s < steps) issue(s);
+    // Fragments of 16 k (two per stage) go through two register sets: one is
+    // read from LDS while the other multiplies.
+    const int fr = lane & 15, fg = lane >> 4;
+    v4f pf[2][TN], qf[2][TM];
+    auto read = [&](int step, auto half) {
+        constexpr int h = decltype(half)::value;
+        const int8_t* st = smem + (step % STAGES) * STAGE_BYTES;
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fa[i] = *reinterpret_cast<const float4*>(&as[s][(wm * 32 + i * 16) * kLdsRow + frag + 16 * half]);
-                fb[i] = *reinterpret_cast<const float4*>(&bs[s][(wn * 32 + i * 16) * kLdsRow + frag + 16 * half]);
-            }
+        for (int i = 0; i < TN; ++i)
+            pf[h][i] = *reinterpret_cast<const v4f*>(st + swz<128>(wn * (TN * 16) + i * 16 + fr, 4 * h + fg));
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < TM; ++j)
+            qf[h][j] = *reinterpret_cast<const v4f*>(st + swz<128>(BN + wm * (TM * 16) + j * 16 + fr, 4 * h + fg));
+    };
+    auto multiply = [&](auto half) {
+        constexpr int h = decltype(half)::value;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i].x, fb[j].x, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i].y, fb[j].y, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i].z, fb[j].z, acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i].w, fb[j].w, acc[i][j], 0, 0, 0);
-                }
-        }
-        // the other stage was last read before the previous barrier
-        if (step + 1 < steps) stash(s ^ 1);
-        __syncthreads();
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[h][i][e], qf[h][j][e], acc[i][j], 0, 0, 0);
+    };
+    // Binary16 operands: both fragments of a stage, rounded, make one
+    // v_mfma_f32_16x16x32_f16 (exact products, fp32 sums). A and B give it
+    // the same k order: lane group fg holds k 4 fg .. + 3 and 16 + 4 fg .. + 3.
+    // Error against 64 bits over the sum of magnitudes, in 2^-24, normal
+    // values: mean 0.12 (K = 768, 3072), largest 1.2; on the fp32 MFMA 0.33
+    // and 3.3. It takes subnormal operands in as multiples of 2^-24 at the
+    // exponent of 2^-14 and sums them with that weight.
+    auto multiply_half = [&] {
+        v8h ph[TN], qh[TM];
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ph[i][e] = static_cast<_Float16>(pf[e >> 2][i][e & 3]);
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qh[j][e] = static_cast<_Float16>(qf[e >> 2][j][e & 3]);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[i], qh[j], acc[i][j], 0, 0, 0);
+    };
+    const std::integral_constant<int, 0> h0;
+    const std::integral_constant<int, 1> h1;
+    wait_stages<STAGES - 1, LPW>(min(STAGES - 1, steps - 1));
+    __builtin_amdgcn_s_barrier();
+    read(0, h0);
+    for (int step = 0; step + 1 < steps; ++step) {
+        read(step, h1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (HALF) multiply_half();
+        else multiply(h0);
+        __builtin_amdgcn_sched_barrier(0);
+        // this wave's operands of the stage are in registers and its copies
+        // of the next stage have landed; after the barrier every wave's have,
+        // and the slot is free for the stage STAGES later
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        wait_stages<STAGES - 2, LPW>(min(STAGES - 2, steps - 2 - step));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (step + STAGES < steps) issue(step + STAGES);
+        read(step + 1, h0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!HALF) multiply(h1);
+    }
+    read(steps - 1, h1);
+    auto clear_past = [&](auto half) {  // k past K (whole chunks, K % 4 == 0): zeros
+        constexpr int h = decltype(half)::value;
+        if (static_cast<uint32_t>(steps - 1) * kBK + 16u * h + 4u * fg < g.k) return;
+#pragma unroll
+        for (int i = 0; i < TN; ++i) pf[h][i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < TM; ++j) qf[h][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+    clear_past(h0);
+    clear_past(h1);
+    if constexpr (HALF) {
+        multiply_half();
+    } else {
+        multiply(h0);
+        multiply(h1);
     }
 
     // 16x16 result layout: lane l holds rows 4 (l / 16) + r of column l % 16.
+    const bool vec = vector_rows<EPI>(g);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < TM; ++j) {
+        const uint32_t m = row0 + wm * (TM * 16) + j * 16 + fr;
+        if (m >= g.m) continue;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t n = col0 + wn * 32 + j * 16 + (lane & 15);
-            if (n >= g.n) continue;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t m = row0 + wm * 32 + i * 16 + 4 * (lane >> 4) + r;
-                if (m < g.m) store_f32<EPI>(g, m, n, acc[i][j][r]);
-            }
+        for (int i = 0; i < TN; ++i) {
+            const uint32_t n = col0 + wn * (TN * 16) + i * 16 + 4 * fg;
+            const float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            if (n < g.n) store_f32<EPI>(g, m, n, v, vec);
         }
+    }
 }
 
 // Native binary16 products: out[m][n] = sum over k = 0, 1, .. K-1 of
@@ -239,15 +349,13 @@ __global__ __launch_bounds__(256) void gemm_h16p_kernel(F32Params g) {
         }
         __syncthreads();
     }
+    const bool vec = vector_rows<EPI>(g);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const uint32_t m = row0 + 4u * ty + r;
         if (m >= g.m) continue;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint32_t n = col0 + 4u * tx + c;
-            if (n < g.n) store_f32<EPI>(g, m, n, s[r][c]);
-        }
+        const uint32_t n = col0 + 4u * tx;
+        if (n < g.n) store_f32<EPI>(g, m, n, s[r], vec);
     }
 }
 
@@ -277,9 +385,74 @@ __global__ __launch_bounds__(256) void im2col_f32_kernel(const float* __restrict
     out[i] = v;
 }
 
+template <int BN, int BM, int WN, int WM, int STAGES, bool HALF, int EPI>
+void launch_tile(const F32Params& g, hipStream_t s) {
+    constexpr size_t lds = static_cast<size_t>(STAGES) * (BN + BM) * 128u;
+    static_assert(lds <= 64u * 1024u, "no larger dynamic LDS is asked for");
+    dispatch(gemm_f32_kernel<BN, BM, WN, WM, STAGES, HALF, EPI>, dim3(ceil_div(g.m, BM), ceil_div(g.n, BN)),
+             dim3(64 * WN * WM), lds, s, g);
+}
+
+constexpr uint32_t kCus = 256;  // MI355X
+
+// float32 operands: the matrix cores bound the time (157 TFLOP/s) and every
+// workgroup of these grids is resident at once, so it goes as the output area
+// of the busiest CU over the rate the tile reaches on a full chip (5480 x
+// 3072 x 1024, TFLOP/s): 93 / 103 / 108 / 109 in the order below. us by that
+// order at 1370 rows, N x K: 4096 x 1024 with GELU 127 / 121 / 132 / 123, 2304
+// x 768 55 / 57 / 58 / 66, 768 x 768 24 / 26 / 24 / 26, 768 x 3072 86 / 97 /
+// 79 / 91.
+template <int EPI>
+void launch_f32(const F32Params& g, hipStream_t s) {
+    struct Tile {
+        uint32_t bn, bm, rate;
+    };
+    constexpr Tile tiles[] = {{32, 32, 93}, {64, 32, 103}, {64, 80, 108}, {64, 96, 109}};
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        if (ceil_div(g.n, tiles[i].bn) > 65535u) continue;  // grid limit; f32_params checked it for 64 columns
+        const uint64_t count = static_cast<uint64_t>(ceil_div(g.n, tiles[i].bn)) * ceil_div(g.m, tiles[i].bm);
+        const double cost = static_cast<double>(ceil_div(count, kCus)) * (tiles[i].bn * tiles[i].bm) / tiles[i].rate;
+        if (best < 0 || cost < least) best = i, least = cost;
+    }
+    switch (best) {
+        case 0: launch_tile<32, 32, 2, 2, 3, false, EPI>(g, s); break;
+        case 1: launch_tile<64, 32, 2, 2, 2, false, EPI>(g, s); break;
+        case 2: launch_tile<64, 80, 4, 1, 2, false, EPI>(g, s); break;
+        default: launch_tile<64, 96, 2, 2, 2, false, EPI>(g, s); break;
+    }
+}
+
+// Binary16 operands: the float32 bytes through L2 and LDS bound the time, so
+// the largest tile that still gives the CUs work. us for 128x128 (8 waves) /
+// 128x64 (8 waves) / 64x64 (four stages) / 32x32 (four stages): 2500 x 3072 x
+// 1024 42 / 54 / 84 / 135 (480 tiles of 128x128), 1370 x 4096 x 1024 with GELU
+// 44 / 40 / 68 / 84 (352; 704 of 128x64), 1370 x 2304 x 768 23 / 21 / 27 / 34
+// (396 of 128x64), 1370 x 768 x 768 21 / 16 / 14 / 16 and 1370 x 768 x 3072
+// 69 / 57 / 40 / 62 (132; 264 of 64x64), 257 x 384 x 384 12 / 9 / 7 / 5 (30).
+// On the float32 MFMA these took 107-190.
+template <int EPI>
+void launch_half(const F32Params& g, hipStream_t s) {
+    auto tiles = [&](uint32_t bn, uint32_t bm) {
+        return static_cast<uint64_t>(ceil_div(g.n, bn)) * ceil_div(g.m, bm);
+    };
+    if (2 * tiles(128, 128) >= 3 * kCus)
+        launch_tile<128, 128, 4, 2, 2, true, EPI>(g, s);
+    else if (tiles(128, 64) >= kCus)
+        launch_tile<128, 64, 4, 2, 2, true, EPI>(g, s);
+    else if (2 * tiles(64, 64) >= kCus)
+        launch_tile<64, 64, 2, 2, 4, true, EPI>(g, s);
+    else
+        launch_tile<32, 32, 2, 2, 4, true, EPI>(g, s);
+}
+
 template <int EPI>
 void launch(const F32Params& g, hipStream_t s) {
-    dispatch(gemm_f32_kernel<EPI>, dim3(ceil_div(g.m, kBM), ceil_div(g.n, kBN)), dim3(256), 0, s, g);
+    if (g.half_operands)
+        launch_half<EPI>(g, s);
+    else
+        launch_f32<EPI>(g, s);
 }
 
 template <int EPI>

@@ -189,44 +189,6 @@ DAV2_DEV void store_one(const GemmParams& g, const EpilogueOperands<EPI, TM, TN>
     g.out[idx] = row_value<EPI, TM, TN>(e, i, j, r, v);
 }
 
-// Waits until at most `later` stages' copies (LPW per stage and wave) are
-// outstanding; later <= MAX (the counts must be immediates).
-template <int MAX, int LPW>
-DAV2_DEV void wait_stages(int later) {
-    if constexpr (MAX <= 0) {
-        DAV2_WAIT_VMCNT(0);
-    } else {
-        if (later >= MAX) DAV2_WAIT_VMCNT(MAX * LPW);
-        else wait_stages<MAX - 1, LPW>(later);
-    }
-}
-
-// Tile index of this workgroup. Workgroups are dealt to the 8 XCDs round
-// robin (id % 8); remap so that each XCD owns one contiguous run of tiles,
-// ordered along M first: the tiles of one weight-column band then share that
-// XCD's L2.
-DAV2_DEV void tile_of(uint32_t& tm, uint32_t& tn) {
-    const uint32_t mt = gridDim.x, total = gridDim.x * gridDim.y;
-    const uint32_t id = blockIdx.y * gridDim.x + blockIdx.x;
-    const uint32_t xcd = id & 7u, idx = id >> 3;
-    const uint32_t base = total >> 3, extra = total & 7u;
-    const uint32_t lin = xcd * base + min(xcd, extra) + idx;
-    tm = lin % mt;
-    tn = lin / mt;
-}
-
-
-// LDS byte offset of logical 16-byte chunk c of row r in a stage of BK-byte
-// rows: chunks are XOR-swizzled with the row's 256-byte period index, so the
-// 16 rows that one MFMA operand load reads at the same logical chunk hit 16
-// distinct bank groups (256 bytes = all banks once).
-template <int BK>
-DAV2_DEV uint32_t swz(uint32_t r, uint32_t c) {
-    constexpr uint32_t cpr = BK / 16, rows_per_period = 256 / BK;
-    return r * BK + ((c ^ ((r / rows_per_period) & (cpr - 1))) << 4);
-}
-
-
 template <int BM, int BN, int WAVES_M, int WAVES_N, int BK, int STAGES, int EPI>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_i8_kernel(GemmParams g) {
     constexpr int NW = WAVES_M * WAVES_N;

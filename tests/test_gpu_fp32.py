@@ -90,6 +90,37 @@ def test_gemm_f32_epilogues(gpu, pkg, lib, oracle, m, n, k, epi):
     assert _rel(got, want) < 1e-5
 
 
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(33, 65, 36), (31, 32, 4), (1297, 2307, 44), (1373, 772, 100), (2443, 3076, 36)])
+def test_gemm_f32_tiles(gpu, pkg, lib, m, n, k, half):
+    """Every tile of both operand forms, ragged in rows, columns and K: within
+    the fp32 sum bound of k terms, binary16 subnormals and overflow included."""
+    torch = gpu
+    _announce("gemm_f32 tiles", m, n, k, half)
+    g = torch.Generator().manual_seed(m + n + k)
+    a, b = torch.randn((m, k), generator=g), torch.randn((n, k), generator=g)
+    a[::7] *= 2.0 ** -20  # binary16 subnormals
+    a[5, 3] = 1.0e5  # past binary16: infinite there, a finite product in fp32
+    ad, bd = a.cuda(), b.cuda()
+    out = torch.full((m, n), float("nan"), device="cuda")
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue, args.out, args.half_operands = m, n, k, 1, ptr(out), half
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    if half:
+        ad, bd = ad.half(), bd.half()
+    want = ad.double() @ bd.double().T
+    # the binary16 MFMA weighs a subnormal operand as one of 2^-14
+    least = 2.0 ** -14 if half else 0.0
+    mag = ad.double().abs().clamp_min(least) @ bd.double().abs().clamp_min(least).T
+    finite = torch.isfinite(want)
+    assert bool((finite[5] == (half == 0)).all())
+    assert torch.equal(out.double()[~finite], want[~finite])
+    # k products (exact for binary16 operands) and k - 1 sums, each within
+    # 2^-24 of its magnitude; 2 k covers both
+    assert bool(((out.double() - want).abs()[finite] <= 2 * k * 2.0 ** -24 * mag[finite]).all())
+
+
 def test_gemm_f32_rejects(gpu, pkg, lib):
     torch = gpu
     a = empty(torch, (8, 8), torch.float32)
