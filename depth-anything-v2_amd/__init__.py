@@ -132,6 +132,12 @@ class ConvArgs(C.Structure):
                 ("partial_in", C.c_void_p), ("partial_out", C.c_void_p)]
 
 
+class ConvF32Args(C.Structure):
+    _fields_ = [("input", C.c_void_p), ("width", C.c_uint32), ("height", C.c_uint32), ("channels", C.c_uint32),
+                ("kernel", C.c_uint32), ("weight", C.c_void_p), ("bias", C.c_void_p), ("out_channels", C.c_uint32),
+                ("flags", C.c_uint32), ("out", C.c_void_p), ("residual", C.c_void_p)]
+
+
 CONV_RELU_INPUT, CONV_RELU_OUTPUT, CONV_EMIT_ABSMAX, CONV_EMIT_RELU_MAX = 1, 2, 4, 8
 
 
@@ -220,6 +226,8 @@ PROTOTYPES = {
     "dav2_hip_gemm_f32": (C.c_int, [C.c_void_p, vp]),
     "dav2_hip_gemm_h16_products": (C.c_int, [C.c_void_p, vp]),
     "dav2_hip_im2col_f32": (C.c_int, [vp, u32, u32, u32, u32, u32, u32, u32, i32, u32, vp, u32, vp]),
+    "dav2_hip_conv2d_f32_supported": (C.c_int, [u32, u32, u32, u32, u32, u32, u32]),
+    "dav2_hip_conv2d_f32": (C.c_int, [C.c_void_p, vp]),
     "dav2_hip_preprocess_bgr8": (C.c_int, [vp, u32, u32, u64, u32, u32, vp, vp]),
     "dav2_hip_preprocess_bgra8_nearest": (C.c_int, [vp, u32, u32, u64, u32, u32, vp, vp]),
     "dav2_hip_normalize_span": (C.c_int, [vp, vp, u64, vp, vp]),

@@ -591,7 +591,8 @@ void HipOperators::project_tokens_float(DeviceBuffer& output, const DeviceBuffer
               "token projection");
 }
 
-// src/operators.cpp:1528-1676: im2col + GEMM, CHW output; fusion as conv2d_int8
+// src/operators.cpp:1528-1676: implicit GEMM, or im2col + GEMM for other
+// geometries; CHW output; fusion as conv2d_int8
 void HipOperators::conv2d(DeviceBuffer& output, const DeviceBuffer& input, const DeviceBuffer& weight,
                           const DeviceBuffer& bias, std::uint32_t input_width, std::uint32_t input_height,
                           std::uint32_t input_channels, std::uint32_t output_channels, std::uint32_t kernel,
@@ -611,6 +612,33 @@ void HipOperators::conv2d(DeviceBuffer& output, const DeviceBuffer& input, const
     require_bytes(output, pixels * output_channels, "convolution output");
     if (fusion.residual) require_bytes(*fusion.residual, pixels * output_channels, "convolution residual");
     const hipStream_t s = stream();
+    // Implicit GEMM, unless the map is small and the channels are many: a few
+    // workgroups then walk all of them one after the other, and the 16-k steps
+    // of the GEMM are the shorter chain (19x19, 768 -> 128: 72 us for im2col +
+    // GEMM, 78 implicit; 37x37, 1024 -> 256: 170 and 127). The output may be
+    // the input's own buffer, which im2col has read before the GEMM writes.
+    const auto at = [](const DeviceBuffer& b) { return reinterpret_cast<std::uintptr_t>(b.data()); };
+    const bool overlaps = at(output) < at(input) + std::uint64_t(input_width) * input_height * input_channels * 4u &&
+                          at(input) < at(output) + pixels * output_channels * 4u;
+    if (dav2_hip_conv2d_f32_supported(input_width, input_height, input_channels, output_channels, kernel, stride,
+                                      padding) &&
+        !overlaps && at(weight) % 16u == 0 && (pixels >= 1024u || input_channels <= 128u)) {
+        dav2_conv_f32_args a{};
+        a.input = input.as<float>();
+        a.width = input_width;
+        a.height = input_height;
+        a.channels = input_channels;
+        a.kernel = kernel;
+        a.weight = weight.as<float>();
+        a.bias = has_bias ? bias.as<float>() : nullptr;
+        a.out_channels = output_channels;
+        a.flags = (fusion.relu_input ? DAV2_CONV_RELU_INPUT : 0u) | (fusion.relu_output ? DAV2_CONV_RELU_OUTPUT : 0u);
+        a.out = output.as<float>();
+        a.residual = fusion.residual ? fusion.residual->as<float>() : nullptr;
+        ProfileScope prof(context_.profiler(), "conv_f32", 2.0 * pixels * output_channels * inner, "OP", s);
+        hip_check(dav2_hip_conv2d_f32(&a, s), "fp32 convolution");
+        return;
+    }
     DeviceBuffer& cols = grow(f32_cols_, pixels * inner * sizeof(float));
     ProfileScope prof_cols(context_.profiler(), "im2col_f32", 4.0 * pixels * inner, "B", s);
     hip_check(dav2_hip_im2col_f32(input.as<float>(), input_width, input_height, input_channels, ow, oh, kernel, stride,

@@ -267,6 +267,28 @@ DAV2_API int dav2_hip_conv_weights_pack(int8_t* dst, const int8_t* src, uint32_t
                                             void* stream);
 DAV2_API int dav2_hip_conv2d_i8(const dav2_conv_i8_args* args, void* stream);
 
+/* Implicit-GEMM fp32 conv2d of the fp32 / fp16 modes (src/operators.cpp:
+ * 1528-1676): kernel 3 / stride 1 / padding 1 with channels % 4 == 0, kernel 1
+ * / stride 1 / padding 0 with channels % 16 == 0
+ * (dav2_hip_conv2d_f32_supported). weight [out_channels][channels*k*k], 16-byte
+ * aligned; flags DAV2_CONV_RELU_INPUT / RELU_OUTPUT; out must not overlap
+ * input (it may be the residual). */
+typedef struct dav2_conv_f32_args {
+    const float* input;          /* CHW [channels][height][width]                  */
+    uint32_t width, height, channels;
+    uint32_t kernel;             /* 1 or 3                                         */
+    const float* weight;
+    const float* bias;           /* [out_channels] or NULL = 0                     */
+    uint32_t out_channels;
+    uint32_t flags;
+    float* out;                  /* CHW [out_channels][height][width]              */
+    const float* residual;       /* NULL, or CHW like out: out = conv + residual   */
+} dav2_conv_f32_args;
+DAV2_API int dav2_hip_conv2d_f32_supported(uint32_t width, uint32_t height, uint32_t channels,
+                                           uint32_t out_channels, uint32_t kernel, uint32_t stride,
+                                           uint32_t padding);
+DAV2_API int dav2_hip_conv2d_f32(const dav2_conv_f32_args* args, void* stream);
+
 /* 1x1 convolution to a few output channels (out_channels <= 4, channels <=
  * 64), the DPT head's last layer (dpt.cpp:838-855 routed through the int8
  * convolution): same bits as dav2_hip_im2col_quantize_i8 + dav2_hip_gemm_i8

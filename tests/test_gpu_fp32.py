@@ -185,6 +185,44 @@ def test_ops_conv2d(gpu, pkg, lib, oracle, ops, c, oc, h, w, k, s, p):
     assert _rel(host(torch, out), oracle.conv2d_f32(x, wt, b, s, p)) < 1e-5
 
 
+@pytest.mark.parametrize("c,oc,h,w,k", [(4, 1, 1, 1, 3), (8, 33, 3, 70, 3), (128, 40, 41, 37, 3), (12, 70, 149, 131, 3),
+                                        (4, 32, 301, 290, 3), (16, 5, 6, 11, 1), (48, 66, 150, 149, 1)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_conv2d_f32_implicit(gpu, pkg, lib, c, oc, h, w, k, fused):
+    """Every tile, ragged in pixels and channels, one-pixel to 301-row maps: the
+    same as float64 within the fp32 sum bound; residual in place, both ReLUs."""
+    torch = gpu
+    _announce("conv2d fp32 implicit", c, oc, h, w, k, fused)
+    g = torch.Generator().manual_seed(c + oc + h)
+    x, wt = torch.randn((c, h, w), generator=g).cuda(), torch.randn((oc, c, k, k), generator=g).cuda()
+    b, res = torch.randn(oc, generator=g).cuda(), torch.randn((oc, h, w), generator=g).cuda()
+    args = pkg.ConvF32Args()
+    args.input, args.width, args.height, args.channels, args.kernel = ptr(x), w, h, c, k
+    args.weight, args.bias, args.out_channels = ptr(wt), ptr(b), oc
+    out = res.clone() if fused else torch.full_like(res, float("nan"))
+    args.out, args.residual, args.flags = ptr(out), ptr(out) if fused else None, 3 if fused else 0
+    ok(lib, lib.dav2_hip_conv2d_f32(C.byref(args), stream(torch)))
+    xin = x.double().relu() if fused else x.double()
+    want = F.conv2d(xin[None].cpu(), wt.double().cpu(), b.double().cpu(), padding=k // 2)[0]
+    mag = F.conv2d(xin.abs()[None].cpu(), wt.double().abs().cpu(), b.double().abs().cpu(), padding=k // 2)[0]
+    if fused:
+        want, mag = (want + res.double().cpu()).relu(), mag + res.double().abs().cpu()
+    # c k k products and as many sums, bias and residual, each within 2^-24 of its magnitude
+    assert bool(((out.double().cpu() - want).abs() <= (2 * c * k * k + 2) * 2.0 ** -24 * mag).all())
+
+
+def test_ops_conv2d_in_place(gpu, pkg, lib, ops):
+    """The output may be the input's buffer (im2col has read it before the GEMM writes)."""
+    torch = gpu
+    g = torch.Generator().manual_seed(1)
+    x, wt, b = torch.randn((16, 9, 70), generator=g), torch.randn((16, 16, 3, 3), generator=g), torch.randn(16)
+    xd, wd, bd = _resident(torch, x.numpy(), wt.numpy(), b.numpy())
+    run(lib, lib.dav2_ops_conv2d(ops, db(pkg, xd), db(pkg, xd), db(pkg, wd), db(pkg, bd), 70, 9, 16, 16, 3, 1, 1, 1))
+    run(lib, lib.dav2_ops_synchronize(ops))
+    want = F.conv2d(x.double()[None], wt.double(), b.double(), padding=1)[0].numpy()
+    assert _rel(host(torch, xd), want) < 1e-5
+
+
 @pytest.mark.parametrize("k", [2, 4])
 def test_ops_conv_transpose(gpu, pkg, lib, oracle, ops, k):
     torch = gpu
