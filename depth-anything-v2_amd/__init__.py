@@ -198,6 +198,7 @@ PROTOTYPES = {
     "dav2_hip_add": (C.c_int, [vp, vp, vp, u64, vp]),
     "dav2_hip_relu": (C.c_int, [vp, vp, u64, vp]),
     "dav2_hip_round_half": (C.c_int, [vp, u64, vp]),
+    "dav2_hip_attention_f32": (C.c_int, [vp, vp, u32, u32, u32, vp]),
     "dav2_hip_attention_scores": (C.c_int, [vp, vp, u32, u32, u32, C.c_int, vp]),
     "dav2_hip_softmax_rows": (C.c_int, [vp, u64, u32, u32, C.c_int, vp]),
     "dav2_hip_attention_values": (C.c_int, [vp, vp, vp, u32, u32, u32, C.c_int, vp]),

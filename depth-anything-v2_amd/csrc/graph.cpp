@@ -80,7 +80,9 @@ void DinoEncoder::forward(const float* image, std::uint32_t width, std::uint32_t
         attention_ == AttentionMode::binary16 || coop ? Precision::fp16 : Precision::fp32;
     DeviceBuffer& scores =
         arena.get("enc.scores", fused ? HipOperators::attention_fused_scratch_bytes(T, H, batch)
-                                      : HipOperators::attention_score_bytes(T, H, batch, materialised));
+                                : precision_ == Precision::fp32
+                                    ? 16  // fused fp32 attention keeps no scores
+                                    : HipOperators::attention_score_bytes(T, H, batch, materialised));
     for (int i = 0; i < 4; ++i) features[i] = &arena.get("enc.feature" + std::to_string(i), tok_bytes);
     // One image: the qkv GEMM also leaves the |k| and |v| column maxima per
     // row tile, so the attention's digit packing reads qkv once.
@@ -165,7 +167,7 @@ void DinoEncoder::forward_fp32(std::uint32_t rows, std::uint32_t T, std::uint32_
     // encoder.cpp:407-597 in the fp32 precision mode: LayerNorm rows in fp32,
     // fp32 GEMMs (GELU and the LayerScale residual in their epilogues, the
     // arithmetic of the reference's separate gelu / add_scaled passes),
-    // materialised fp32 attention. The fp16 mode (encoder.cpp:428-546): the
+    // fused fp32 attention. The fp16 mode (encoder.cpp:428-546): the
     // same with the GEMM operands rounded to binary16 (layer_norm_fp16 and
     // pack_fp16 produce binary16 inputs, fc1's output is stored as binary16
     // and fc2 reads it) and the reference's binary16 attention, or its fp32
@@ -181,7 +183,7 @@ void DinoEncoder::forward_fp32(std::uint32_t rows, std::uint32_t T, std::uint32_
         ops_.linear_f32(qkv, normed, W(".attn.qkv.weight"), &W(".attn.qkv.bias"), rows, D, 3 * D, E::row, nullptr, 0,
                         half);
         if (!half)
-            ops_.attention_mfma_f32(attn, qkv, T, H, batch, scores);
+            ops_.attention_mfma_f32(attn, qkv, T, H, batch);
         else
             ops_.attention_batched(attn, qkv, T, H, batch, scores,
                                    attention_ == AttentionMode::fp32 ? Precision::fp32 : Precision::fp16,

@@ -355,29 +355,11 @@ void HipOperators::attention_batched(DeviceBuffer& output, const DeviceBuffer& q
 }
 
 void HipOperators::attention_mfma_f32(DeviceBuffer& output, const DeviceBuffer& qkv, std::uint32_t tokens,
-                                      std::uint32_t heads, std::uint32_t batch, DeviceBuffer& scores) {
-    if (scores.size() < dav2_hip_attention_scratch_bytes(tokens, heads, batch, 0))
-        throw std::invalid_argument("attention score scratch device buffer is too small");
+                                      std::uint32_t heads, std::uint32_t batch) {
     const hipStream_t s = stream();
-    const double flops = 2.0 * batch * heads * double(tokens) * tokens * 64.0;
-    const double score_bytes = double(batch) * heads * tokens * tokens * 4.0;
-    Profiler& prof = context_.profiler();
-    {
-        ProfileScope p(prof, "attention_scores", flops, "FLOP", s);
-        hip_check(dav2_hip_attention_scores(scores.data(), qkv.as<float>(), tokens, heads, batch, 0, s),
-                  "attention scores");
-    }
-    {
-        ProfileScope p(prof, "softmax_f32_mfma_path", 2.0 * score_bytes, "B", s);
-        hip_check(dav2_hip_softmax_rows(scores.data(), std::uint64_t(batch) * heads * tokens, tokens, tokens, 0, s),
-                  "attention softmax");
-    }
-    {
-        ProfileScope p(prof, "attention_values", flops, "FLOP", s);
-        hip_check(dav2_hip_attention_values(output.as<float>(), scores.data(), qkv.as<float>(), tokens, heads, batch,
-                                            0, s),
-                  "attention values");
-    }
+    const double flops = 4.0 * batch * heads * double(tokens) * tokens * 64.0;
+    ProfileScope p(context_.profiler(), "attention_f32", flops, "FLOP", s);
+    hip_check(dav2_hip_attention_f32(output.as<float>(), qkv.as<float>(), tokens, heads, batch, s), "attention");
 }
 
 std::uint64_t HipOperators::attention_fused_scratch_bytes(std::uint32_t tokens, std::uint32_t heads,

@@ -224,10 +224,10 @@ public:
                            Precision precision, bool cooperative = false);
     static std::uint64_t attention_score_bytes(std::uint32_t tokens, std::uint32_t heads, std::uint32_t batch,
                                                Precision precision);
-    // fp32 attention on the matrix cores (fp32 precision mode): the same
-    // scratch as attention_batched(fp32), sums in the MFMA's own order.
+    // fp32 attention on the matrix cores (fp32 precision mode), fused: no
+    // score buffer, sums in the MFMA's own order.
     void attention_mfma_f32(DeviceBuffer& output, const DeviceBuffer& qkv, std::uint32_t tokens,
-                            std::uint32_t heads, std::uint32_t batch, DeviceBuffer& scores);
+                            std::uint32_t heads, std::uint32_t batch);
     // Fused integer-exact attention (int8 digit planes, exact int32 MFMA
     // sums): the int8-mode default in place of the materialised binary16
     // scores.

@@ -314,8 +314,14 @@ DAV2_API int dav2_hip_relu(float* out, const float* input, uint64_t count, void*
  * (src/gpu_model.cpp:51-98) applied on the device. */
 DAV2_API int dav2_hip_round_half(float* data, uint64_t count, void* stream);
 
-/* fp32 attention, head_dim 64, on the matrix cores (the fp32 precision
- * mode's path; src/operators.cpp:1169-1208 with bmm.glsl and
+/* fp32 attention, head_dim 64, fused (the fp32 precision mode's path): scores,
+ * softmax and values in one kernel, no score buffer, sums in the MFMA's order. qkv and
+ * out [batch*T][H*64] 16-byte aligned. */
+DAV2_API int dav2_hip_attention_f32(float* out, const float* qkv, uint32_t tokens, uint32_t heads,
+                                    uint32_t batch, void* stream);
+
+/* fp32 attention, head_dim 64, on the matrix cores over materialised scores
+ * (src/operators.cpp:1169-1208 with bmm.glsl and
  * softmax_lastdim.glsl, sums in the MFMA's order: within tolerance of the
  * reference, not bit for bit). qkv is [batch*T][3*H*64] token-major (q | k |
  * v, head h at h*64); scores [batch][H][T][T] fp32, softmax in place,

@@ -761,6 +761,41 @@ def _attention_ref_gpu(torch, lib, qkv, tokens, heads, fp16, batch=1, unpacked=T
     return host(torch, out), probs, scores
 
 
+@pytest.mark.parametrize("tokens,heads,batch,sigma", [(1, 1, 1, 1.0), (15, 2, 1, 1.0), (31, 1, 3, 2.0), (32, 1, 1, 1.0),
+                                                      (33, 2, 1, 1.0), (64, 1, 1, 4.0), (65, 3, 2, 1.0),
+                                                      (97, 1, 1, 1.0), (545, 6, 2, 3.0), (1370, 2, 1, 1.2),
+                                                      (2443, 1, 1, 2.0)])
+def test_attention_f32_fused(gpu, lib, tokens, heads, batch, sigma):
+    # against float64 attention. A score's error is about 64 roundings of
+    # magnitudes up to sum |q k| / 8, and it scales its weight by as much; the
+    # weighted sum adds at most about sqrt(T) roundings of sum p |v|.
+    torch = gpu
+    _announce("fused fp32 attention", tokens, heads, batch)
+    rng = np.random.default_rng(tokens + heads)
+    qkv = (rng.standard_normal((batch * tokens, 3 * heads * 64)) * sigma).astype(np.float32)
+    qd = dev(torch, qkv)
+    out = empty(torch, (batch * tokens, heads * 64), torch.float32)
+    ok(lib, lib.dav2_hip_attention_f32(ptr(out), ptr(qd), tokens, heads, batch, stream(torch)))
+    got = host(torch, out).reshape(batch, tokens, heads, 64)
+    x = qkv.astype(np.float64).reshape(batch, tokens, 3, heads, 64)
+    for b in range(batch):
+        for h in range(heads):
+            q, k, v = x[b, :, 0, h] * 0.125, x[b, :, 1, h], x[b, :, 2, h]
+            s = q @ k.T
+            p = np.exp(s - s.max(axis=1, keepdims=True))
+            p /= p.sum(axis=1, keepdims=True)
+            score_err = 8.0 * 2.0 ** -24 * (np.abs(q) @ np.abs(k).T).max(axis=1)
+            bound = (p @ np.abs(v)) * (2.0 * score_err[:, None] + (16.0 + np.sqrt(tokens)) * 2.0 ** -24)
+            assert np.all(np.abs(got[b, :, h] - p @ v) <= bound + 1e-30)
+    # NaN in one query row stays in that row; infinite values behind the last token do not exist
+    if tokens > 1 and batch == 1:
+        qd[0, 0] = float("nan")
+        ok(lib, lib.dav2_hip_attention_f32(ptr(out), ptr(qd), tokens, heads, batch, stream(torch)))
+        again = host(torch, out).reshape(tokens, heads, 64)
+        assert np.all(np.isnan(again[0, 0])) and np.array_equal(again[1:], got[0, 1:])
+    assert lib.dav2_hip_attention_f32(0, ptr(qd), tokens, heads, batch, stream(torch)) != 0
+
+
 @pytest.mark.parametrize("tokens,heads,batch", [(1, 1, 1), (5, 2, 1), (65, 3, 1), (258, 2, 2), (1370, 6, 1),
                                                 (1370, 16, 1)])
 def test_attention_ref_fp32_bit_exact(gpu, lib, oracle, tokens, heads, batch):
