@@ -1,7 +1,7 @@
 // fp32 and fp16 paths of the precision modes (DAV2_CREATE_FORCE_FP32 /
 // FORCE_FP16): the linear and convolution GEMMs in float32 on the MFMA
-// (v_mfma_f32_16x16x4_f32; v_mfma_f32_16x16x32_f16 on operands rounded to
-// binary16), with the epilogues of the int8 GEMM, and the fp32 im2col that
+// (v_mfma_f32_16x16x4_f32, or v_mfma_f32_16x16x32_bf16 on operands split in
+// three; v_mfma_f32_16x16x32_f16 on operands rounded to binary16), with the epilogues of the int8 GEMM, and the fp32 im2col that
 // feeds convolutions.
 //
 // fp16 arithmetic comes in the reference's two forms. Cooperative-matrix
@@ -288,6 +288,179 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
     }
 }
 
+typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
+// Four floats as three bfloat16 parts each, x = part 0 + part 1 + part 2
+// exactly (8 significant bits each, cut off and not rounded).
+DAV2_DEV void split_bf16(v4f x, v2u (&part)[3]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint32_t u[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) u[e] = __float_as_uint(x[e]);
+        part[k] = v2u{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)};
+        if (k < 2)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] -= __uint_as_float(u[e] & 0xFFFF0000u);
+    }
+}
+
+// fp32 operands on the bfloat16 MFMA: each operand is split into three parts
+// on its way into LDS (global -> registers, two stages ahead -> three planes of
+// 64-byte rows) and six products per element, all but those of 2^-24 and below,
+// go to v_mfma_f32_16x16x32_bf16, smallest first: 96 matrix cycles for 32 k of a
+// block where v_mfma_f32_16x16x4_f32 takes 256. Relative error against 64 bits
+// over K = 384 .. 4096: 0.84 - 0.9 of the fp32 MFMA's (6.5e-7 -> 5.6e-7 at K =
+// 1024). What bounds it: LDS (four plane reads and one write for each product of
+// a 32x32 wave block) and the VALU's splitting.
+template <int BN, int BM, int WN, int WM, int EPI>
+__global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
+    constexpr int NT = 64 * WN * WM, TN = BN / WN / 16, TM = BM / WM / 16;
+    constexpr int ROWS = BN + BM, LPT = ROWS * 8 / NT;  // float4 loads per thread and stage
+    constexpr int PLANE = ROWS * 64, STAGE = 3 * PLANE;  // bytes
+    static_assert(TN * WN * 16 == BN && TM * WM * 16 == BM && LPT * NT == ROWS * 8, "whole blocks and loads");
+    extern __shared__ __attribute__((aligned(16))) int8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave / WM, wm = wave % WM;
+    const int fr = lane & 15, fg = lane >> 4;
+    uint32_t tm, tn;
+    tile_of(tm, tn);
+    const uint32_t row0 = tm * BM, col0 = tn * BN;
+    const int steps = static_cast<int>((g.k + kBK - 1) / kBK);
+
+    // Thread t's load i is float4 t % 8 of stage row t / 8 + i NT / 8. Rows
+    // past the matrix read its last row (never stored), k past K is zero.
+    const uint32_t kq = 4u * (tid & 7);
+    const float* src[LPT];
+    uint32_t dst[LPT];
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+        const uint32_t r = (tid >> 3) + i * (NT / 8);
+        src[i] = (r < static_cast<uint32_t>(BN) ? g.b + min(col0 + r, g.n - 1) * g.ldb
+                                                : g.a + min(row0 + r - BN, g.m - 1) * g.lda) + kq;
+        dst[i] = swz<64>(r, (tid & 7) >> 1) + 8u * (tid & 1);
+    }
+    v4f next[2][LPT];
+    auto load = [&](int step, auto set) {
+        const bool in = static_cast<uint32_t>(step) * kBK + kq < g.k;
+#pragma unroll
+        for (int i = 0; i < LPT; ++i) {
+            next[decltype(set)::value][i] = *reinterpret_cast<const v4f*>(src[i] + (in ? step * kBK : -static_cast<int>(kq)));
+        }
+    };
+    auto stash = [&](int step, auto set) {
+        const bool in = static_cast<uint32_t>(step) * kBK + kq < g.k;
+        int8_t* st = smem + decltype(set)::value * STAGE;
+#pragma unroll
+        for (int i = 0; i < LPT; ++i) {
+            v2u part[3];
+            split_bf16(in ? next[decltype(set)::value][i] : v4f{0.f, 0.f, 0.f, 0.f}, part);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<v2u*>(st + k * PLANE + dst[i]) = part[k];
+        }
+    };
+
+    v4f acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    const std::integral_constant<int, 0> h0;
+    const std::integral_constant<int, 1> h1;
+    load(0, h0);
+    load(min(1, steps - 1), h1);
+    stash(0, h0);
+    load(min(2, steps - 1), h0);
+    __syncthreads();
+    auto stage = [&](int step, auto cur, auto nxt) {
+        const int8_t* st = smem + decltype(cur)::value * STAGE;
+        v8b pf[3][TN], qf[3][TM];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+                pf[k][i] = *reinterpret_cast<const v8b*>(st + k * PLANE + swz<64>(wn * (TN * 16) + i * 16 + fr, fg));
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+                qf[k][j] = *reinterpret_cast<const v8b*>(st + k * PLANE + swz<64>(BN + wm * (TM * 16) + j * 16 + fr, fg));
+        }
+        // unconditional (past the last stage it is loaded again and never
+        // read), so that the waits count the other set's loads as in flight
+        stash(step + 1, nxt);
+        load(min(step + 3, steps - 1), nxt);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int pp[6] = {2, 1, 0, 1, 0, 0}, qq[6] = {0, 1, 2, 0, 1, 0};  // smallest products first
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[pp[t]][i], qf[qq[t]][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+    };
+    int step = 0;
+    for (; step + 1 < steps; step += 2) {
+        stage(step, h0, h1);
+        stage(step + 1, h1, h0);
+    }
+    if (step < steps) stage(step, h0, h1);
+
+    // An infinite operand splits into NaN parts: a wave that ends with a NaN
+    // sums its block again on the fp32 MFMA, operands straight from memory.
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) nan |= acc[i][j][r] != acc[i][j][r];
+    if (__any(nan)) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (uint32_t k = 4u * fg; k < g.k + 4u * fg; k += 16u) {
+            v4f p[TN], q[TM];
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const uint32_t n = min(col0 + wn * (TN * 16) + i * 16 + fr, g.n - 1);
+                p[i] = k < g.k ? *reinterpret_cast<const v4f*>(g.b + n * g.ldb + k) : v4f{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int j = 0; j < TM; ++j) {
+                const uint32_t m = min(row0 + wm * (TM * 16) + j * 16 + fr, g.m - 1);
+                q[j] = k < g.k ? *reinterpret_cast<const v4f*>(g.a + m * g.lda + k) : v4f{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TM; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][e], q[j][e], acc[i][j], 0, 0, 0);
+        }
+    }
+
+    // 16x16 result layout: lane l holds rows 4 (l / 16) + r of column l % 16.
+    const bool vec = vector_rows<EPI>(g);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const uint32_t m = row0 + wm * (TM * 16) + j * 16 + fr;
+        if (m >= g.m) continue;
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+            const uint32_t n = col0 + wn * (TN * 16) + i * 16 + 4 * fg;
+            const float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+            if (n < g.n) store_f32<EPI>(g, m, n, v, vec);
+        }
+    }
+}
+
 // Native binary16 products: out[m][n] = sum over k = 0, 1, .. K-1 of
 // float(fp16(h(a[m][k]) * h(b[n][k]))) in fp32, h = round to binary16, then
 // the epilogue (+ bias): prepare_tokens_fp16.glsl:37-52,
@@ -402,8 +575,25 @@ constexpr uint32_t kCus = 256;  // MI355X
 // order at 1370 rows, N x K: 4096 x 1024 with GELU 127 / 121 / 132 / 123, 2304
 // x 768 55 / 57 / 58 / 66, 768 x 768 24 / 26 / 24 / 26, 768 x 3072 86 / 97 /
 // 79 / 91.
+//
+// From 512 tiles of 128x64 on (two for every CU) the bfloat16 split of 128x64
+// on 8 waves: us against the best of the above at rows x N x K 1370 x 4096 x
+// 1024 with GELU 101 / 138, 1814 x 3072 x 768 72 / 98, 1814 x 2304 x 768 66 /
+// 73, 5480 x 3072 x 1024 256 / 330; below that it does not fill the chip (1814 x
+// 768 x 3072 93-98 / 93, 1370 x 1024 x 1024 40 / 38), nor do its 64x64 (32x32)
+// tiles beat the above (43, 49).
 template <int EPI>
 void launch_f32(const F32Params& g, hipStream_t s) {
+    constexpr uint32_t kBn = 128, kBm = 64;
+    constexpr size_t lds = 2u * 3u * (kBn + kBm) * 64u;
+    static const bool roomy =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<kBn, kBm, 4, 2, EPI>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess;
+    if (roomy && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus) {
+        dispatch(gemm_split_kernel<kBn, kBm, 4, 2, EPI>, dim3(ceil_div(g.m, kBm), ceil_div(g.n, kBn)), dim3(512), lds,
+                 s, g);
+        return;
+    }
     struct Tile {
         uint32_t bn, bm, rate;
     };

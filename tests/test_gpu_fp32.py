@@ -121,6 +121,32 @@ def test_gemm_f32_tiles(gpu, pkg, lib, m, n, k, half):
     assert bool(((out.double() - want).abs()[finite] <= 2 * k * 2.0 ** -24 * mag[finite]).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(2000, 2100, 4), (2017, 2049, 32), (1985, 2177, 68), (2500, 2052, 100)])
+def test_gemm_f32_split(gpu, pkg, lib, m, n, k):
+    """Grids that take the bfloat16 split: magnitudes over 40 binades within the
+    bound of test_gemm_f32_tiles (the three parts are exact and the products
+    left out below 3 x 2^-24 of their magnitude), infinities and NaN as in fp32."""
+    torch = gpu
+    _announce("gemm_f32 split", m, n, k)
+    g = torch.Generator().manual_seed(m + n + k)
+    a, b = torch.randn((m, k), generator=g), torch.randn((n, k), generator=g)
+    a[::7] *= 2.0 ** -20
+    b[::5] *= 2.0 ** 20
+    a[5, 3], a[70, 2], b[9, 3], a[131, 1] = float("inf"), float("nan"), 0.0, -float("inf")
+    ad, bd = a.cuda(), b.cuda()
+    out = torch.full((m, n), 7.0, device="cuda")
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue, args.out = m, n, k, 1, ptr(out)
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    want = ad.double() @ bd.double().T
+    finite = torch.isfinite(want)
+    assert not bool(finite[5].any()) and not bool(finite[70].any()) and int((~finite).sum()) == 3 * n
+    assert torch.equal(out[~finite].nan_to_num(1.0, 2.0, 3.0).double(), want[~finite].nan_to_num(1.0, 2.0, 3.0))
+    mag = ad.double().abs() @ bd.double().abs().T
+    assert bool(((out.double() - want).abs()[finite] <= (2 * k + 3) * 2.0 ** -24 * mag[finite]).all())
+
+
 def test_gemm_f32_rejects(gpu, pkg, lib):
     torch = gpu
     a = empty(torch, (8, 8), torch.float32)
