@@ -638,30 +638,6 @@ __global__ __launch_bounds__(256) void ref_values_kernel(float* __restrict__ out
 // sum += float(a16 * b16) at 1.5 VALU instructions per product.
 constexpr uint32_t kChunkWords = 32u * 64u;  // one 64-token chunk of keys or values
 
-// acc = acc + float(lo(prod)), one IEEE fp32 addition (the binary16 half
-// widened exactly, times 1.0, plus acc: v_fma_mix_f32 rounds once).
-DAV2_DEV void add_product_lo(float& acc, uint32_t prod, float one) {
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(prod), "v"(one));
-}
-// acc = acc + float(hi(prod))
-DAV2_DEV void add_product_hi(float& acc, uint32_t prod, float one) {
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(prod), "v"(one));
-}
-
-// acc[n] = (acc[n] + float(lo(prod[n]))) + float(hi(prod[n])) for N sums;
-// the low halves of all N first, so that dependent additions are N apart.
-template <int N>
-DAV2_DEV void add_product_pairs(float (&acc)[N], const uint32_t (&prod)[N], float one) {
-#pragma unroll
-    for (int n = 0; n < N; ++n) add_product_lo(acc[n], prod[n], one);
-#pragma unroll
-    for (int n = 0; n < N; ++n) add_product_hi(acc[n], prod[n], one);
-}
-
-DAV2_DEV uint32_t mul_half2(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, a) * __builtin_bit_cast(h2, b));
-}
-
 __global__ __launch_bounds__(256) void ref16_pack_kernel(const float* __restrict__ qkv, uint32_t* __restrict__ k16,
                                                          uint32_t* __restrict__ v16, uint32_t tokens, uint32_t heads,
                                                          uint32_t chunks) {

@@ -39,8 +39,7 @@ namespace {
 
 using namespace dav2k;
 
-constexpr int kBM = 64, kBN = 64;  // gemm_h16p_kernel's tile
-constexpr int kBK = 32;            // floats per K step
+constexpr int kBK = 32;  // floats per K step
 
 struct F32Params {
     const float* a;
@@ -466,69 +465,96 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
 // the epilogue (+ bias): prepare_tokens_fp16.glsl:37-52,
 // project_tokens_common.glsl (NATIVE_FP16) and
 // conv_transpose_nonoverlap_common.glsl (NATIVE_FP16), whose sums run over
-// the inner index in ascending order. Thread (tx, ty) of 16 x 16 owns rows
-// 4 ty .. +3 and columns 4 tx .. +3 of a 64 x 64 tile; K goes in chunks of
-// 32, staged k-major in LDS as binary16 values held in floats (exact).
-template <int EPI>
+// the inner index in ascending order.
+//
+// Bounded by the VALU (a product is half a v_pk_mul_f16, two k at once, and a
+// v_fma_mix_f32 that widens and adds it) and, since every sum is one chain over
+// K, by the waves that hide its latency: small tiles, 32 R x 32 on four waves.
+// Thread t owns rows t / 8 (+ 32) and columns 4 (t % 8) .. + 3. K goes in
+// chunks of 64, rounded on the way from registers (one chunk ahead) into one of
+// two LDS buffers of 128-byte rows, whose 16-byte pieces (8 k) are XOR-swizzled
+// so that the rows a wave reads at once fall on different banks. Past K both
+// operands are zero: + 0 leaves a sum as it is.
+// us at rows x N x K, 64x64 tiles of 4x4 a thread and the products widened and
+// added separately -> this: 1369 x 768 x 588 131 -> 57, 1369 x 96 x 768 122 ->
+// 21, 1369 x 768 x 768 166 -> 66, 5476 x 1024 x 1024 527 -> 331 (17 T
+// products/s), 252 x 384 x 588 94 -> 18.
+constexpr uint32_t kMaxGridY = 65535u;
+
+template <int R, int EPI>
 __global__ __launch_bounds__(256) void gemm_h16p_kernel(F32Params g) {
-    __shared__ __attribute__((aligned(16))) float as[kBK][kBM + 4];
-    __shared__ __attribute__((aligned(16))) float bs[kBK][kBN + 4];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const uint32_t row0 = blockIdx.x * kBM, col0 = blockIdx.y * kBN;
-    float s[4][4];
+    constexpr int kRows = 32 * R + 32, kLoads = kRows * 16 / 256;  // columns (weights) first
+    __shared__ __attribute__((aligned(16))) int8_t tile[2][kRows * 128];
+    const uint32_t tid = threadIdx.x, tx = tid & 7u, ty = tid >> 3;
+    const uint32_t row0 = blockIdx.x * 32u * R, col0 = (blockIdx.z * kMaxGridY + blockIdx.y) * 32u;
+    if (col0 >= g.n) return;
+    auto piece = [](uint32_t r, uint32_t c) { return r * 128u + ((c ^ r ^ (r >> 2)) & 7u) * 16u; };
+
+    // Thread t's load i is float4 t % 16 of tile row t / 16 + 16 i; rows past
+    // the matrix read its last row (never stored).
+    const uint32_t kq = 4u * (tid & 15u);
+    const float* src[kLoads];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int i = 0; i < kLoads; ++i) {
+        const uint32_t r = (tid >> 4) + 16u * i;
+        src[i] = i < 2 ? g.b + min(col0 + r, g.n - 1) * g.ldb : g.a + min(row0 + r - 32u, g.m - 1) * g.lda;
+    }
+    v4f next[kLoads];
+    auto load = [&](uint32_t k0) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) next[i] = *reinterpret_cast<const v4f*>(src[i] + (k0 + kq < g.k ? k0 + kq : 0u));
+    };
+    auto stash = [&](uint32_t k0, int8_t* buf) {
+        const bool in = k0 + kq < g.k;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) {
+            const v4f v = in ? next[i] : v4f{0.f, 0.f, 0.f, 0.f};
+            const v4h h = {static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]), static_cast<_Float16>(v[2]),
+                           static_cast<_Float16>(v[3])};
+            *reinterpret_cast<v4h*>(buf + piece((tid >> 4) + 16u * i, (tid & 15u) >> 1) + 8u * (tid & 1u)) = h;
+        }
+    };
+
+    float s[R][4];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int c = 0; c < 4; ++c) s[r][c] = 0.0f;
-    for (uint32_t k0 = 0; k0 < g.k; k0 += kBK) {
-        // float4 idx = tid + 256 i of each 64 x 32 operand tile: row idx / 8,
-        // k 4 (idx % 8) .. +3 (K is a multiple of 4)
+    const float one = 1.0f;
+    load(0);
+    stash(0, tile[0]);
+    load(64u);
+    for (uint32_t k0 = 0, buf = 0; k0 < g.k; k0 += 64u, buf ^= 1u) {
+        __syncthreads();  // this chunk is in LDS; every wave is done with the other buffer
+        stash(k0 + 64u, tile[buf ^ 1u]);
+        load(k0 + 128u);
+        const int8_t* t = tile[buf];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = tid + 256 * i;
-            const uint32_t r = static_cast<uint32_t>(idx >> 3), kq = 4u * (idx & 7), kk = k0 + kq;
-            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-            const float4 va = row0 + r < g.m && kk < g.k
-                                  ? *reinterpret_cast<const float4*>(g.a + static_cast<uint64_t>(row0 + r) * g.lda + kk)
-                                  : zero;
-            const float4 vb = col0 + r < g.n && kk < g.k
-                                  ? *reinterpret_cast<const float4*>(g.b + static_cast<uint64_t>(col0 + r) * g.ldb + kk)
-                                  : zero;
-            as[kq + 0][r] = round_half(va.x);
-            as[kq + 1][r] = round_half(va.y);
-            as[kq + 2][r] = round_half(va.z);
-            as[kq + 3][r] = round_half(va.w);
-            bs[kq + 0][r] = round_half(vb.x);
-            bs[kq + 1][r] = round_half(vb.y);
-            bs[kq + 2][r] = round_half(vb.z);
-            bs[kq + 3][r] = round_half(vb.w);
-        }
-        __syncthreads();
-        const uint32_t kc = min(static_cast<uint32_t>(kBK), g.k - k0);  // no terms past K
-#pragma unroll 4
-        for (uint32_t k = 0; k < kc; ++k) {
-            const float4 av = *reinterpret_cast<const float4*>(&as[k][ty * 4]);
-            const float4 bv = *reinterpret_cast<const float4*>(&bs[k][tx * 4]);
-            const h2 b01 = {static_cast<_Float16>(bv.x), static_cast<_Float16>(bv.y)};
-            const h2 b23 = {static_cast<_Float16>(bv.z), static_cast<_Float16>(bv.w)};
-            const float a[4] = {av.x, av.y, av.z, av.w};
+        for (uint32_t c8 = 0; c8 < 8; ++c8) {
+            uint4 av[R], bv[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const _Float16 ah = static_cast<_Float16>(a[r]);
-                const h2 aa = {ah, ah};
-                add_half_products(s[r][0], s[r][1], aa, b01);
-                add_half_products(s[r][2], s[r][3], aa, b23);
+            for (int r = 0; r < R; ++r) av[r] = *reinterpret_cast<const uint4*>(t + piece(32u + 32u * r + ty, c8));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) bv[c] = *reinterpret_cast<const uint4*>(t + piece(4u * tx + c, c8));
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                auto word = [p](const uint4& v) { return p == 0 ? v.x : p == 1 ? v.y : p == 2 ? v.z : v.w; };
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    uint32_t prod[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) prod[c] = mul_half2(word(av[r]), word(bv[c]));
+                    add_product_pairs(s[r], prod, one);
+                }
             }
         }
-        __syncthreads();
     }
     const bool vec = vector_rows<EPI>(g);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const uint32_t m = row0 + 4u * ty + r;
-        if (m >= g.m) continue;
+    for (int r = 0; r < R; ++r) {
+        const uint32_t m = row0 + 32u * r + ty;
         const uint32_t n = col0 + 4u * tx;
-        if (n < g.n) store_f32<EPI>(g, m, n, s[r], vec);
+        if (m < g.m && n < g.n) store_f32<EPI>(g, m, n, s[r], vec);
     }
 }
 
@@ -647,7 +673,14 @@ void launch(const F32Params& g, hipStream_t s) {
 
 template <int EPI>
 void launch_h16p(const F32Params& g, hipStream_t s) {
-    dispatch(gemm_h16p_kernel<EPI>, dim3(ceil_div(g.m, kBM), ceil_div(g.n, kBN)), dim3(256), 0, s, g);
+    const uint32_t nt = ceil_div(g.n, 32);
+    const dim3 cols(0, min(nt, kMaxGridY), ceil_div(nt, kMaxGridY));
+    // two rows a thread halve the LDS reads of a product, one row gives twice
+    // the waves: us at 5476 x 1024 x 1024 331 / 354, 1369 x 768 x 768 74 / 66
+    if (static_cast<uint64_t>(ceil_div(g.m, 64)) * nt >= 8u * kCus)
+        dispatch(gemm_h16p_kernel<2, EPI>, dim3(ceil_div(g.m, 64), cols.y, cols.z), dim3(256), 0, s, g);
+    else
+        dispatch(gemm_h16p_kernel<1, EPI>, dim3(ceil_div(g.m, 32), cols.y, cols.z), dim3(256), 0, s, g);
 }
 
 // Checks a dav2_gemm_f32_args and fills the kernel parameters; false if the
@@ -655,7 +688,7 @@ void launch_h16p(const F32Params& g, hipStream_t s) {
 bool f32_params(const dav2_gemm_f32_args* a, F32Params& g) {
     if (!a || !a->a || !a->b || !a->out || a->m == 0 || a->n == 0 || a->k == 0 || a->k % 4u || a->lda < a->k ||
         a->ldb < a->k || a->lda % 4u || a->ldb % 4u || (reinterpret_cast<uintptr_t>(a->a) & 15u) ||
-        (reinterpret_cast<uintptr_t>(a->b) & 15u) || ceil_div(a->n, kBN) > 65535u || a->half_operands > 1u)
+        (reinterpret_cast<uintptr_t>(a->b) & 15u) || ceil_div(a->n, 64) > 65535u || a->half_operands > 1u)
         return false;
     const uint32_t e = a->epilogue;
     if (e != DAV2_GEMM_EPI_ROW && e != DAV2_GEMM_EPI_ROW_GELU && e != DAV2_GEMM_EPI_ROW_LAYERSCALE &&

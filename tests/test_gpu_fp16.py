@@ -71,6 +71,13 @@ def test_gemm_h16_products_bit_exact(gpu, pkg, lib, oracle, m, n, k, epi):
         f"{np.count_nonzero(got.view(np.uint32) != want.view(np.uint32))} of {got.size} differ"
 
 
+@pytest.mark.parametrize("m,n,k,epi", [(33, 31, 60, "row"), (65, 36, 64, "transposed"), (31, 33, 132, "row"),
+                                       (32, 32, 192, "transposed"), (2081, 1996, 68, "row")])
+def test_gemm_h16_products_tile_edges(gpu, pkg, lib, oracle, m, n, k, epi):
+    # tile and K chunk remainders, both tile heights
+    test_gemm_h16_products_bit_exact(gpu, pkg, lib, oracle, m, n, k, epi)
+
+
 def test_gemm_h16_products_rejects(gpu, pkg, lib):
     torch = gpu
     a = torch.zeros((4, 8), dtype=torch.float32, device="cuda")
