@@ -130,6 +130,124 @@ __global__ __launch_bounds__(kBlock) void bilinear_kernel(float* __restrict__ ou
     if (CPT == 32 && maxima) maxima[static_cast<uint64_t>(blockIdx.z) * oplane + static_cast<uint64_t>(oy) * ow + ox] = m;
 }
 
+// Upsampling (oh >= ih): a wave walks kStripRows output rows of 64 columns and
+// 8 channels and keeps the two horizontally blended source rows between them, so
+// that a source value is loaded once or twice (each output of bilinear_kernel
+// loads four), the next source row's loads in flight; the same operations on the
+// same values. The four waves take neighbouring tiles, or with maxima (channels %
+// 32 == 0) the 32 channels of one, and then write max |out| of them. Workgroups
+// are numbered so that each XCD takes a contiguous run of the map: neighbouring
+// row pieces, which share cache lines, meet in one L2.
+//
+// Bound by the stores to memory (3 TB/s with the reads; the stores are scattered
+// over 8 planes). us on buffers out of the caches, bilinear_kernel -> this: 296 ->
+// 518, 128 channels 61.5 -> 57.7, with maxima 68.9 -> 61.2; 148 -> 296, 256 channels
+// 40.8 -> 37.0, with maxima 45.2 -> 39.1. Strips of 8 or 16 rows: the same on large
+// maps, 1-5 us slower on small ones; nontemporal stores 60-68.
+constexpr uint32_t kStripRows = 4;
+
+template <bool MAX>
+__global__ __launch_bounds__(kBlock) void bilinear_up_kernel(float* __restrict__ out, const float* __restrict__ in,
+                                                             uint32_t iw, uint32_t ih, uint32_t ow, uint32_t oh,
+                                                             uint32_t channels, uint32_t tiles_x, uint32_t tiles_y,
+                                                             float* __restrict__ maxima) {
+    constexpr uint32_t C = 8;
+    __shared__ float peak[MAX ? kBlock / 64 : 1][kStripRows][64];
+    const uint32_t total = gridDim.x, xcd = blockIdx.x & 7u, per = total >> 3, extra = total & 7u;
+    const uint32_t lin = xcd * per + min(xcd, extra) + (blockIdx.x >> 3);
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tiles = tiles_x * tiles_y, per_group = MAX ? tiles : (tiles + 3u) / 4u;
+    const uint32_t group = lin / per_group;
+    const uint32_t tile = MAX ? lin - group * per_group : (lin - group * per_group) * 4u + wave;
+    const uint32_t ty = tile / tiles_x;
+    const uint32_t ox = (tile - ty * tiles_x) * 64u + lane, oy0 = ty * kStripRows;
+    const uint32_t c0 = MAX ? group * 32u + wave * C : group * C;
+    const uint32_t n = c0 < channels && oy0 < oh ? min(C, channels - c0) : 0u;
+    const uint64_t iplane = static_cast<uint64_t>(ih) * iw, oplane = static_cast<uint64_t>(oh) * ow;
+    if (n != 0u) {
+        const uint32_t xc = min(ox, ow - 1u);
+        const float sx = ow > 1 ? static_cast<float>(xc) * static_cast<float>(iw - 1) / static_cast<float>(ow - 1) : 0.0f;
+        const uint32_t x0 = static_cast<uint32_t>(floorf(sx));
+        const uint32_t x1 = min(x0 + 1u, iw - 1u);
+        const float fx = sx - static_cast<float>(x0);
+        auto source_row = [&](uint32_t oy, float& fy) {
+            const float sy = oh > 1 ? static_cast<float>(oy) * static_cast<float>(ih - 1) / static_cast<float>(oh - 1) : 0.0f;
+            const float y0 = floorf(sy);
+            fy = sy - y0;
+            return __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(y0));
+        };
+        const float* src = in + static_cast<uint64_t>(c0) * iplane;
+        float a[C], b[C], top[C], bottom[C];
+        auto load = [&](uint32_t y) {
+            const float* row = src + static_cast<uint64_t>(min(y, ih - 1u)) * iw;
+#pragma unroll
+            for (uint32_t k = 0; k < C; ++k) {
+                const float* p = row + static_cast<uint64_t>(min(k, n - 1u)) * iplane;  // clamped: every load valid
+                a[k] = p[x0];
+                b[k] = p[x1];
+            }
+        };
+        auto blend = [&](float (&row)[C]) {
+#pragma unroll
+            for (uint32_t k = 0; k < C; ++k) row[k] = a[k] * (1.0f - fx) + b[k] * fx;
+        };
+        float fy;
+        uint32_t y = source_row(oy0, fy);
+        load(y);
+        blend(top);
+        load(y + 1u);
+        blend(bottom);
+        load(y + 2u);
+        float* dst = out + static_cast<uint64_t>(c0) * oplane + static_cast<uint64_t>(oy0) * ow + ox;
+#pragma unroll
+        for (uint32_t j = 0; j < kStripRows; ++j) {
+            if (oy0 + j >= oh) break;
+            const uint32_t y0 = source_row(oy0 + j, fy);
+            while (y < y0) {  // uniform; once at most per row where oh >= ih
+#pragma unroll
+                for (uint32_t k = 0; k < C; ++k) top[k] = bottom[k];
+                blend(bottom);
+                ++y;
+                load(y + 2u);
+            }
+            float m = 0.0f;
+#pragma unroll
+            for (uint32_t k = 0; k < C; ++k) {
+                const float v = top[k] * (1.0f - fy) + bottom[k] * fy;
+                if (k < n && ox < ow) dst[static_cast<uint64_t>(k) * oplane + static_cast<uint64_t>(j) * ow] = v;
+                m = fmaxf(m, fabsf(v));
+            }
+            if (MAX) peak[wave][j][lane] = m;
+        }
+    }
+    if constexpr (!MAX) return;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kStripRows * 64u; i += kBlock) {
+        const uint32_t j = i >> 6, l = i & 63u, x = (tile - ty * tiles_x) * 64u + l;
+        if (oy0 + j < oh && x < ow)
+            maxima[static_cast<uint64_t>(group) * oplane + static_cast<uint64_t>(oy0 + j) * ow + x] =
+                fmaxf(fmaxf(peak[0][j][l], peak[1][j][l]), fmaxf(peak[2][j][l], peak[3][j][l]));
+    }
+}
+
+// Below 4 Mi outputs the plain resize has more waves for its one round trip (us
+// at 37 -> 74, 256 channels 5.1 / 5.4, 74 -> 148 10.0 / 8.6); with the maxima this
+// one is faster from there too (6.5 / 5.4, 11.3 / 8.8), its waves sharing the 32
+// channels. Fewer output rows than input rows would load rows no output needs.
+template <bool MAX>
+bool launch_bilinear_up(float* out, float* partial, const float* input, uint32_t iw, uint32_t ih, uint32_t ow,
+                        uint32_t oh, uint32_t channels, hipStream_t s) {
+    const uint32_t tx = ceil_div(ow, 64), ty = ceil_div(oh, kStripRows);
+    const uint64_t tiles = static_cast<uint64_t>(tx) * ty;
+    const uint64_t groups = MAX ? tiles * (channels / 32u) : (tiles + 3u) / 4u * ceil_div(channels, 8);
+    if (oh < ih || groups > 0xffffffu) return false;
+    if (!MAX && static_cast<uint64_t>(ow) * oh * channels < (4u << 20)) return false;
+    dispatch(bilinear_up_kernel<MAX>, dim3(static_cast<uint32_t>(groups)), dim3(kBlock), 0, s, out, input, iw, ih, ow,
+             oh, channels, tx, ty, partial);
+    return true;
+}
+
 // reduce_minmax.glsl as a grid reduction. Stage 1: each workgroup folds a
 // grid-stride slice into one (min, max) pair; stage 2: one workgroup folds the
 // partials. min/max are exact, so the result does not depend on the order.
@@ -318,6 +436,8 @@ int dav2_hip_bilinear_align_true(float* out, const float* input, uint32_t iw, ui
                                  uint32_t oh, uint32_t channels, void* stream) {
     if (ow == 0 || oh == 0 || channels == 0) return hipSuccess;
     if (!out || !input || iw == 0 || ih == 0 || channels > 65535u) return hipErrorInvalidValue;
+    if (launch_bilinear_up<false>(out, nullptr, input, iw, ih, ow, oh, channels, static_cast<hipStream_t>(stream)))
+        return hipGetLastError();
     const dim3 grid(ceil_div(ow, 64), ceil_div(oh, 4), ceil_div(channels, kBilinearChannels));
     dispatch(bilinear_kernel<kBilinearChannels>, grid, dim3(kBlock), 0, static_cast<hipStream_t>(stream),
                        out, input, iw, ih, ow, oh, channels, nullptr);
@@ -329,6 +449,8 @@ int dav2_hip_bilinear_align_true_maxima(float* out, float* partial, const float*
     if (ow == 0 || oh == 0 || channels == 0) return hipSuccess;
     if (!out || !partial || !input || iw == 0 || ih == 0 || channels % 32u || channels > 65535u)
         return hipErrorInvalidValue;
+    if (launch_bilinear_up<true>(out, partial, input, iw, ih, ow, oh, channels, static_cast<hipStream_t>(stream)))
+        return hipGetLastError();
     const dim3 grid(ceil_div(ow, 64), ceil_div(oh, 4), channels / 32u);
     dispatch(bilinear_kernel<32>, grid, dim3(kBlock), 0, static_cast<hipStream_t>(stream), out, input, iw,
                        ih, ow, oh, channels, partial);

@@ -1300,6 +1300,13 @@ def test_bilinear_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow):
     assert np.array_equal(host(torch, out).view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("c,ih,iw,oh,ow", [(13, 201, 300, 599, 601), (35, 130, 350, 130, 950), (70, 1, 9, 241, 259),
+                                           (66, 127, 3, 1001, 65)])
+def test_bilinear_strips_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow):
+    # from 4 Mi outputs on: ragged strips, tiles and channel groups, one source row, equal heights
+    test_bilinear_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow)
+
+
 @pytest.mark.parametrize("n", [4, 1000, 518 * 518, 1036 * 1036 + 5])
 def test_minmax_normalize(gpu, lib, oracle, n):
     torch = gpu
