@@ -604,12 +604,26 @@ constexpr uint32_t kWideTileRows = 4096;
 // Columns of Q from which those GEMMs take 128x128 tiles on eight waves.
 constexpr uint32_t kWideTileCols = 3072;
 
-// Rows of P per tile of the configuration launch_epi picks: 128 / 64 for the
+// Rows of P per tile of the configuration launch_epi picks, for the epilogue
+// with column maxima (the others take 32 in few_tiles grids): 128 / 64 for the
 // 128x128 / 64x128 tiles of the large row-major GEMMs without column maxima
 // (rows_p >= kWideTileRows), else 32, 96 or 64 as in the switch below.
 // Columns of Q from which the smaller row-major GEMMs without column maxima
 // (fc1 at batch 1) take 128x64 tiles on eight waves.
 constexpr uint32_t kTallTileCols = 4096;
+
+// Grids of at most one 64x64 tile a CU leave most of the chip idle while a
+// few waves walk K: 32x32 tiles on four waves (the column maxima, whose row
+// tiles the caller has counted, keep 64x64 and take eight waves). us at rows x N x K, 64x64 -> 32x32: 253 x 384 x 384
+// LayerScale 4.2 -> 3.3, 253 x 384 x 1536 7.8 -> 7.0, 253 x 1536 x 384 GELU 6.3 ->
+// 4.1, 252 x 384 x 384 channel-major 5.6 -> 3.7, 61 x 1024 x 4096 15.4 -> 11.9,
+// 545 x 768 x 768 (108 tiles) 5.7 -> 4.8, 1370 x 384 x 1536 (132) 8.0 -> 7.2; 1370
+// x 768 x 3072 (264) 15.7 -> 15.9, 1370 x 1024 x 1024 (352) 8.1 -> 8.7. Eight
+// waves: 253 x 1152 x 384 5.0 -> 4.1. Six stages in place of three: 0.2-0.5
+// slower but for the longest K.
+inline bool few_tiles(uint32_t rows_p, uint32_t rows_q, uint32_t slices) {
+    return static_cast<uint64_t>(ceil_div(rows_p, 64)) * ceil_div(rows_q, 64) * slices <= 256u;
+}
 
 inline uint32_t tile_rows(uint32_t rows_p, uint32_t rows_q, bool row_major, bool col_max) {
     if (row_major && !col_max && rows_p >= kWideTileRows) return rows_q >= kWideTileCols ? 128 : 64;
@@ -656,6 +670,15 @@ void launch_epi(const GemmParams& g, hipStream_t s, bool last = true) {
         }
         if (g.rows_q >= kTallTileCols && g.rows_p >= 512) {
             launch_cfg<128, 64, 4, 2, 128, 2, EPI>(g, s, last);
+            return;
+        }
+    }
+    if (few_tiles(g.rows_p, g.rows_q, ceil_div(g.k, g.k_split))) {
+        if constexpr (EPI != DAV2_GEMM_EPI_ROW_COLMAX) {
+            launch_cfg<32, 32, 2, 2, 128, 3, EPI>(g, s, last);
+            return;
+        } else if (g.rows_p > 32 && (g.rows_q < 2048 || g.rows_p < 512)) {  // tile_rows: 64
+            launch_cfg<64, 64, 4, 2, 128, 4, EPI>(g, s, last);
             return;
         }
     }

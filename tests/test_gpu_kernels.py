@@ -531,6 +531,15 @@ def test_gemm_row_epilogues(gpu, pkg, lib, oracle, m, n, k):
     assert np.array_equal(host(torch, outr).view(np.uint32), refr.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,n,k", [(31, 33, 64), (33, 65, 192), (1024, 1024, 128), (1025, 1024, 128), (253, 1536, 384)])
+def test_gemm_few_tiles(gpu, pkg, lib, oracle, m, n, k):
+    # up to one 64x64 tile a CU takes 32x32 tiles: edges of both and of the rule
+    test_gemm_row_epilogues(gpu, pkg, lib, oracle, m, n, k)
+    test_gemm_transposed_residual_relu(gpu, pkg, lib, oracle, m, n, k)
+    if n % 64 == 0:
+        test_gemm_colmax_epilogue(gpu, pkg, lib, oracle, m, n, k, n - 64)
+
+
 @pytest.mark.parametrize("m,n,k,begin", [(1370, 3072, 1024, 1024), (1369, 2304, 384, 768), (300, 1024, 256, 512),
                                          (20, 192, 64, 64), (1, 128, 64, 0)])
 def test_gemm_colmax_epilogue(gpu, pkg, lib, oracle, m, n, k, begin):
