@@ -470,7 +470,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
 // Bounded by the VALU (a product is half a v_pk_mul_f16, two k at once, and a
 // v_fma_mix_f32 that widens and adds it) and, since every sum is one chain over
 // K, by the waves that hide its latency: small tiles, 32 R x 32 on four waves.
-// Thread t owns rows t / 8 (+ 32) and columns 4 (t % 8) .. + 3. K goes in
+// A thread owns one row (or two, 32 apart) of 32 and four columns. K goes in
 // chunks of 64, rounded on the way from registers (one chunk ahead) into one of
 // two LDS buffers of 128-byte rows, whose 16-byte pieces (8 k) are XOR-swizzled
 // so that the rows a wave reads at once fall on different banks. Past K both
@@ -485,7 +485,9 @@ template <int R, int EPI>
 __global__ __launch_bounds__(256) void gemm_h16p_kernel(F32Params g) {
     constexpr int kRows = 32 * R + 32, kLoads = kRows * 16 / 256;  // columns (weights) first
     __shared__ __attribute__((aligned(16))) int8_t tile[2][kRows * 128];
-    const uint32_t tid = threadIdx.x, tx = tid & 7u, ty = tid >> 3;
+    // channel-major epilogues store along the rows: there the lanes run over them
+    constexpr bool kAlongRows = EPI == DAV2_GEMM_EPI_CONVT || EPI == DAV2_GEMM_EPI_TRANSPOSED;
+    const uint32_t tid = threadIdx.x, tx = kAlongRows ? tid >> 5 : tid & 7u, ty = kAlongRows ? tid & 31u : tid >> 3;
     const uint32_t row0 = blockIdx.x * 32u * R, col0 = (blockIdx.z * kMaxGridY + blockIdx.y) * 32u;
     if (col0 >= g.n) return;
     auto piece = [](uint32_t r, uint32_t c) { return r * 128u + ((c ^ r ^ (r >> 2)) & 7u) * 16u; };
