@@ -1,15 +1,15 @@
 // fp32 and fp16 paths of the precision modes (DAV2_CREATE_FORCE_FP32 /
 // FORCE_FP16): the linear and convolution GEMMs in float32 on the MFMA
 // (v_mfma_f32_16x16x4_f32, or v_mfma_f32_16x16x32_bf16 on operands split in
-// three; v_mfma_f32_16x16x32_f16 on operands rounded to binary16), with the epilogues of the int8 GEMM, and the fp32 im2col that
-// feeds convolutions.
+// three), with the epilogues of the int8 GEMM, and the fp32 im2col that feeds
+// convolutions.
 //
 // fp16 arithmetic comes in the reference's two forms. Cooperative-matrix
 // linears (linear_coop_fp16.glsl via linear_fp16* with cooperative_matrix_fp16,
 // src/operators.cpp:540-768): operands rounded to binary16, exact products,
 // fp32 accumulation. The fp32 GEMM does this with half_operands: both operands
-// are rounded to binary16 on their way from LDS to v_mfma_f32_16x16x32_f16,
-// whose products are exact and whose sums are fp32. Native binary16 shaders
+// are rounded to binary16 on their way from LDS to v_mfma_f32_16x16x4_f32, which
+// multiplies them exactly and sums in fp32. Native binary16 shaders
 // (prepare_tokens_fp16, project_tokens_fp16, conv_transpose_nonoverlap_fp16):
 // every product is a binary16 multiplication, widened and added to an fp32 sum
 // in k order; gemm_h16p_kernel does exactly that on the VALU, so its results
@@ -198,38 +198,26 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
         for (int j = 0; j < TM; ++j)
             qf[h][j] = *reinterpret_cast<const v4f*>(st + swz<128>(BN + wm * (TM * 16) + j * 16 + fr, 4 * h + fg));
     };
+    // Binary16 operands are rounded here; the fp32 MFMA's products of them are
+    // exact, subnormal ones included (v_mfma_f32_16x16x32_f16 sums a subnormal
+    // operand with the weight of one of 2^-14).
+    auto operand = [](v4f v) {
+        return HALF ? __builtin_convertvector(__builtin_convertvector(v, v4h), v4f) : v;
+    };
     auto multiply = [&](auto half) {
         constexpr int h = decltype(half)::value;
+        v4f p[TN], q[TM];
+#pragma unroll
+        for (int i = 0; i < TN; ++i) p[i] = operand(pf[h][i]);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) q[j] = operand(qf[h][j]);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll
                 for (int j = 0; j < TM; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[h][i][e], qf[h][j][e], acc[i][j], 0, 0, 0);
-    };
-    // Binary16 operands: both fragments of a stage, rounded, make one
-    // v_mfma_f32_16x16x32_f16 (exact products, fp32 sums). A and B give it
-    // the same k order: lane group fg holds k 4 fg .. + 3 and 16 + 4 fg .. + 3.
-    // Error against 64 bits over the sum of magnitudes, in 2^-24, normal
-    // values: mean 0.12 (K = 768, 3072), largest 1.2; on the fp32 MFMA 0.33
-    // and 3.3. It takes subnormal operands in as multiples of 2^-24 at the
-    // exponent of 2^-14 and sums them with that weight.
-    auto multiply_half = [&] {
-        v8h ph[TN], qh[TM];
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ph[i][e] = static_cast<_Float16>(pf[e >> 2][i][e & 3]);
-#pragma unroll
-        for (int j = 0; j < TM; ++j)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qh[j][e] = static_cast<_Float16>(qf[e >> 2][j][e & 3]);
-#pragma unroll
-        for (int i = 0; i < TN; ++i)
-#pragma unroll
-            for (int j = 0; j < TM; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph[i], qh[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][e], q[j][e], acc[i][j], 0, 0, 0);
     };
     const std::integral_constant<int, 0> h0;
     const std::integral_constant<int, 1> h1;
@@ -238,10 +226,11 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
     read(0, h0);
     for (int step = 0; step + 1 < steps; ++step) {
         read(step, h1);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (HALF) multiply_half();
-        else multiply(h0);
-        __builtin_amdgcn_sched_barrier(0);
+        // rounding and products of binary16 operands interleave freely
+        // (1370 x 2304 x 768 70 -> 65 us)
+        if constexpr (!HALF) __builtin_amdgcn_sched_barrier(0);
+        multiply(h0);
+        if constexpr (!HALF) __builtin_amdgcn_sched_barrier(0);
         // this wave's operands of the stage are in registers and its copies
         // of the next stage have landed; after the barrier every wave's have,
         // and the slot is free for the stage STAGES later
@@ -252,7 +241,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
         if (step + STAGES < steps) issue(step + STAGES);
         read(step + 1, h0);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!HALF) multiply(h1);
+        multiply(h1);
     }
     read(steps - 1, h1);
     auto clear_past = [&](auto half) {  // k past K (whole chunks, K % 4 == 0): zeros
@@ -265,12 +254,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
     };
     clear_past(h0);
     clear_past(h1);
-    if constexpr (HALF) {
-        multiply_half();
-    } else {
-        multiply(h0);
-        multiply(h1);
-    }
+    multiply(h0);
+    multiply(h1);
 
     // 16x16 result layout: lane l holds rows 4 (l / 16) + r of column l % 16.
     const bool vec = vector_rows<EPI>(g);
@@ -596,14 +581,38 @@ void launch_tile(const F32Params& g, hipStream_t s) {
 
 constexpr uint32_t kCus = 256;  // MI355X
 
-// float32 operands: the matrix cores bound the time (157 TFLOP/s) and every
-// workgroup of these grids is resident at once, so it goes as the output area
-// of the busiest CU over the rate the tile reaches on a full chip (5480 x
-// 3072 x 1024, TFLOP/s): 93 / 103 / 108 / 109 in the order below. us by that
-// order at 1370 rows, N x K: 4096 x 1024 with GELU 127 / 121 / 132 / 123, 2304
-// x 768 55 / 57 / 58 / 66, 768 x 768 24 / 26 / 24 / 26, 768 x 3072 86 / 97 /
-// 79 / 91.
-//
+// The fp32 MFMA bounds the time (157 TFLOP/s) and every workgroup of these
+// grids is resident at once, so it goes as the output area of the busiest CU
+// over the rate the tile reaches on a full chip (5480 x 3072 x 1024, TFLOP/s):
+// 93 / 103 / 108 / 109 in the order below, on operands that are rounded to
+// binary16 on the way 76 / 91 / 100 / 107. us by that order at 1370 rows, N x
+// K, float32: 4096 x 1024 with GELU 127 / 121 / 132 / 123, 2304 x 768 55 / 57 /
+// 58 / 66, 768 x 768 24 / 26 / 24 / 26, 768 x 3072 86 / 97 / 79 / 91; binary16:
+// 4096 x 1024 158 / 130 / 138 / 122, 2304 x 768 73 / 65 / 66 / 71, 768 x 768 32 /
+// 32 / 30 / 30, 768 x 3072 115 / 114 / 107 / 108.
+template <bool HALF, int EPI>
+void launch_tiles(const F32Params& g, hipStream_t s) {
+    struct Tile {
+        uint32_t bn, bm, rate;
+    };
+    constexpr Tile tiles[] = {{32, 32, HALF ? 76 : 93}, {64, 32, HALF ? 91 : 103}, {64, 80, HALF ? 100 : 108},
+                              {64, 96, HALF ? 107 : 109}};
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        if (ceil_div(g.n, tiles[i].bn) > 65535u) continue;  // grid limit; f32_params checked it for 64 columns
+        const uint64_t count = static_cast<uint64_t>(ceil_div(g.n, tiles[i].bn)) * ceil_div(g.m, tiles[i].bm);
+        const double cost = static_cast<double>(ceil_div(count, kCus)) * (tiles[i].bn * tiles[i].bm) / tiles[i].rate;
+        if (best < 0 || cost < least) best = i, least = cost;
+    }
+    switch (best) {
+        case 0: launch_tile<32, 32, 2, 2, HALF ? 4 : 3, HALF, EPI>(g, s); break;
+        case 1: launch_tile<64, 32, 2, 2, 2, HALF, EPI>(g, s); break;
+        case 2: launch_tile<64, 80, 4, 1, 2, HALF, EPI>(g, s); break;
+        default: launch_tile<64, 96, 2, 2, 2, HALF, EPI>(g, s); break;
+    }
+}
+
 // From 512 tiles of 128x64 on (two for every CU) the bfloat16 split of 128x64
 // on 8 waves: us against the best of the above at rows x N x K 1370 x 4096 x
 // 1024 with GELU 101 / 138, 1814 x 3072 x 768 72 / 98, 1814 x 2304 x 768 66 /
@@ -617,58 +626,17 @@ void launch_f32(const F32Params& g, hipStream_t s) {
     static const bool roomy =
         hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<kBn, kBm, 4, 2, EPI>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess;
-    if (roomy && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus) {
+    if (roomy && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus)
         dispatch(gemm_split_kernel<kBn, kBm, 4, 2, EPI>, dim3(ceil_div(g.m, kBm), ceil_div(g.n, kBn)), dim3(512), lds,
                  s, g);
-        return;
-    }
-    struct Tile {
-        uint32_t bn, bm, rate;
-    };
-    constexpr Tile tiles[] = {{32, 32, 93}, {64, 32, 103}, {64, 80, 108}, {64, 96, 109}};
-    int best = -1;
-    double least = 0.0;
-    for (int i = 0; i < 4; ++i) {
-        if (ceil_div(g.n, tiles[i].bn) > 65535u) continue;  // grid limit; f32_params checked it for 64 columns
-        const uint64_t count = static_cast<uint64_t>(ceil_div(g.n, tiles[i].bn)) * ceil_div(g.m, tiles[i].bm);
-        const double cost = static_cast<double>(ceil_div(count, kCus)) * (tiles[i].bn * tiles[i].bm) / tiles[i].rate;
-        if (best < 0 || cost < least) best = i, least = cost;
-    }
-    switch (best) {
-        case 0: launch_tile<32, 32, 2, 2, 3, false, EPI>(g, s); break;
-        case 1: launch_tile<64, 32, 2, 2, 2, false, EPI>(g, s); break;
-        case 2: launch_tile<64, 80, 4, 1, 2, false, EPI>(g, s); break;
-        default: launch_tile<64, 96, 2, 2, 2, false, EPI>(g, s); break;
-    }
-}
-
-// Binary16 operands: the float32 bytes through L2 and LDS bound the time, so
-// the largest tile that still gives the CUs work. us for 128x128 (8 waves) /
-// 128x64 (8 waves) / 64x64 (four stages) / 32x32 (four stages): 2500 x 3072 x
-// 1024 42 / 54 / 84 / 135 (480 tiles of 128x128), 1370 x 4096 x 1024 with GELU
-// 44 / 40 / 68 / 84 (352; 704 of 128x64), 1370 x 2304 x 768 23 / 21 / 27 / 34
-// (396 of 128x64), 1370 x 768 x 768 21 / 16 / 14 / 16 and 1370 x 768 x 3072
-// 69 / 57 / 40 / 62 (132; 264 of 64x64), 257 x 384 x 384 12 / 9 / 7 / 5 (30).
-// On the float32 MFMA these took 107-190.
-template <int EPI>
-void launch_half(const F32Params& g, hipStream_t s) {
-    auto tiles = [&](uint32_t bn, uint32_t bm) {
-        return static_cast<uint64_t>(ceil_div(g.n, bn)) * ceil_div(g.m, bm);
-    };
-    if (2 * tiles(128, 128) >= 3 * kCus)
-        launch_tile<128, 128, 4, 2, 2, true, EPI>(g, s);
-    else if (tiles(128, 64) >= kCus)
-        launch_tile<128, 64, 4, 2, 2, true, EPI>(g, s);
-    else if (2 * tiles(64, 64) >= kCus)
-        launch_tile<64, 64, 2, 2, 4, true, EPI>(g, s);
     else
-        launch_tile<32, 32, 2, 2, 4, true, EPI>(g, s);
+        launch_tiles<false, EPI>(g, s);
 }
 
 template <int EPI>
 void launch(const F32Params& g, hipStream_t s) {
     if (g.half_operands)
-        launch_half<EPI>(g, s);
+        launch_tiles<true, EPI>(g, s);
     else
         launch_f32<EPI>(g, s);
 }
