@@ -275,28 +275,47 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
 typedef __bf16 v8b __attribute__((ext_vector_type(8)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
-// Four floats as three bfloat16 parts each, x = part 0 + part 1 + part 2
-// exactly (8 significant bits each, cut off and not rounded).
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2b __attribute__((ext_vector_type(2)));
+
+// Operands are split times 2^24: the parts of anything above 2^-126 are then
+// normal bfloat16 values, and those of subnormal floats too. Past 2^103 they
+// are infinite, as are sums past 2^80.
+constexpr float kSplitScale = 16777216.0f;
+
+// Four floats as three bfloat16 parts each, every part the value nearest to
+// what is left (ties to even): x = part 0 + part 1 + part 2 exactly, |part 1| <=
+// 2^-8 and |part 2| <= 2^-17 of the power of two at or below |x|.
 DAV2_DEV void split_bf16(v4f x, v2u (&part)[3]) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        uint32_t u[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) u[e] = __float_as_uint(x[e]);
-        part[k] = v2u{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)};
-        if (k < 2)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] -= __uint_as_float(u[e] & 0xFFFF0000u);
+        for (int h = 0; h < 2; ++h) {
+            const v2f pair = {x[2 * h], x[2 * h + 1]};
+            const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, v2b));
+            part[k][h] = u;
+            if (k < 2) {
+                x[2 * h] -= __uint_as_float(u << 16);
+                x[2 * h + 1] -= __uint_as_float(u & 0xFFFF0000u);
+            }
+        }
     }
 }
 
 // fp32 operands on the bfloat16 MFMA: each operand is split into three parts
 // on its way into LDS (global -> registers, two stages ahead -> three planes of
-// 64-byte rows) and six products per element, all but those of 2^-24 and below,
-// go to v_mfma_f32_16x16x32_bf16, smallest first: 96 matrix cycles for 32 k of a
-// block where v_mfma_f32_16x16x4_f32 takes 256. Relative error against 64 bits
-// over K = 384 .. 4096: 0.84 - 0.9 of the fp32 MFMA's (6.5e-7 -> 5.6e-7 at K =
-// 1024). What bounds it: LDS (four plane reads and one write for each product of
+// 64-byte rows) and six products per element go to v_mfma_f32_16x16x32_bf16: 96
+// matrix cycles for 32 k of a block where v_mfma_f32_16x16x4_f32 takes 256. The
+// three left out (parts 1 and 2, twice, and 2 and 2) are at most (1 + 2^-10)
+// 2^-24 of the element's product. Products of the same order (part numbers that
+// add up to 0, 1, 2) have a sum of their own: the MFMA cuts off what lies below
+// its accumulator, and the small products added to the large sum cost 10 times
+// this error where all operands are positive. Relative error against 64 bits,
+// fp32 MFMA -> this, K = 64 / 384 / 1024 / 4096: normal operands 1.4e-7 / 3.5e-7 /
+// 5.7e-7 / 1.1e-6 -> 5.0e-8 / 1.1e-7 / 1.9e-7 / 4.0e-7, positive ones 1.2e-7 / 2.7e-7
+// / 4.9e-7 / 9.9e-7 -> 5.2e-8 / 1.0e-7 / 1.8e-7 / 3.5e-7, mantissas of the largest
+// left-out products 9.3e-8 / 2.1e-7 / 5.2e-7 / 8.8e-6 -> 6.2e-8 / 6.6e-8 / 6.2e-8 /
+// 6.8e-8. What bounds it: LDS (four plane reads and one write for each product of
 // a 32x32 wave block) and the VALU's splitting.
 template <int BN, int BM, int WN, int WM, int EPI>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
@@ -340,17 +359,17 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
 #pragma unroll
         for (int i = 0; i < LPT; ++i) {
             v2u part[3];
-            split_bf16(in ? next[decltype(set)::value][i] : v4f{0.f, 0.f, 0.f, 0.f}, part);
+            split_bf16(in ? next[decltype(set)::value][i] * kSplitScale : v4f{0.f, 0.f, 0.f, 0.f}, part);
 #pragma unroll
             for (int k = 0; k < 3; ++k) *reinterpret_cast<v2u*>(st + k * PLANE + dst[i]) = part[k];
         }
     };
 
-    v4f acc[TN][TM];
+    v4f acc[TN][TM], mid[TN][TM], low[TN][TM];  // sums of the products of order 0, 1, 2
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TM; ++j) acc[i][j] = mid[i][j] = low[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     const std::integral_constant<int, 0> h0;
     const std::integral_constant<int, 1> h1;
@@ -376,14 +395,17 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
         stash(step + 1, nxt);
         load(min(step + 3, steps - 1), nxt);
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int pp[6] = {2, 1, 0, 1, 0, 0}, qq[6] = {0, 1, 2, 0, 1, 0};  // smallest products first
+        constexpr int pp[6] = {2, 1, 0, 1, 0, 0}, qq[6] = {0, 0, 0, 1, 1, 2};
 #pragma unroll
         for (int t = 0; t < 6; ++t)
 #pragma unroll
             for (int i = 0; i < TN; ++i)
 #pragma unroll
-                for (int j = 0; j < TM; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[pp[t]][i], qf[qq[t]][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TM; ++j) {
+                    const int order = pp[t] + qq[t];
+                    v4f& sum = order == 0 ? acc[i][j] : order == 1 ? mid[i][j] : low[i][j];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[pp[t]][i], qf[qq[t]][j], sum, 0, 0, 0);
+                }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
     };
@@ -394,20 +416,26 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
     }
     if (step < steps) stage(step, h0, h1);
 
-    // An infinite operand splits into NaN parts: a wave that ends with a NaN
-    // sums its block again on the fp32 MFMA, operands straight from memory.
-    bool nan = false;
+    // Infinite and NaN operands, and operands and sums that the scale takes past
+    // the largest float, end as infinities or NaN here: a wave with such a sum
+    // computes its block again on the fp32 MFMA, operands straight from memory,
+    // and takes those sums from there.
+    auto infinite = [](float v) { return !(fabsf(v) <= 3.402823466e+38f); };
+    bool again = false;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
         for (int j = 0; j < TM; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) nan |= acc[i][j][r] != acc[i][j][r];
-    if (__any(nan)) {
+            for (int r = 0; r < 4; ++r) {
+                acc[i][j][r] = (acc[i][j][r] + (mid[i][j][r] + low[i][j][r])) * (1.0f / (kSplitScale * kSplitScale));
+                again |= infinite(acc[i][j][r]);
+            }
+    if (__any(again)) {
 #pragma unroll
         for (int i = 0; i < TN; ++i)
 #pragma unroll
-            for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < TM; ++j) mid[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
         for (uint32_t k = 4u * fg; k < g.k + 4u * fg; k += 16u) {
             v4f p[TN], q[TM];
 #pragma unroll
@@ -426,8 +454,15 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
                 for (int i = 0; i < TN; ++i)
 #pragma unroll
                     for (int j = 0; j < TM; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][e], q[j][e], acc[i][j], 0, 0, 0);
+                        mid[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[i][e], q[j][e], mid[i][j], 0, 0, 0);
         }
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (infinite(acc[i][j][r])) acc[i][j][r] = mid[i][j][r];
     }
 
     // 16x16 result layout: lane l holds rows 4 (l / 16) + r of column l % 16.
@@ -619,6 +654,12 @@ void launch_tiles(const F32Params& g, hipStream_t s) {
 // 73, 5480 x 3072 x 1024 256 / 330; below that it does not fill the chip (1814 x
 // 768 x 3072 93-98 / 93, 1370 x 1024 x 1024 40 / 38), nor do its 64x64 (32x32)
 // tiles beat the above (43, 49).
+//
+// Below K = 64 the products the split leaves out can cost more than the sums of
+// the fp32 MFMA: 6.2e-8 against 3.3e-8 / 6.1e-8 / 7.7e-8 / 9.3e-8 at K = 8 / 32 / 48
+// / 64 for operands chosen for it.
+constexpr uint32_t kSplitDepth = 64;
+
 template <int EPI>
 void launch_f32(const F32Params& g, hipStream_t s) {
     constexpr uint32_t kBn = 128, kBm = 64;
@@ -626,7 +667,7 @@ void launch_f32(const F32Params& g, hipStream_t s) {
     static const bool roomy =
         hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<kBn, kBm, 4, 2, EPI>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess;
-    if (roomy && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus)
+    if (roomy && g.k >= kSplitDepth && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus)
         dispatch(gemm_split_kernel<kBn, kBm, 4, 2, EPI>, dim3(ceil_div(g.m, kBm), ceil_div(g.n, kBn)), dim3(512), lds,
                  s, g);
     else

@@ -121,9 +121,10 @@ def test_gemm_f32_tiles(gpu, pkg, lib, m, n, k, half):
 
 @pytest.mark.parametrize("m,n,k", [(2000, 2100, 4), (2017, 2049, 32), (1985, 2177, 68), (2500, 2052, 100)])
 def test_gemm_f32_split(gpu, pkg, lib, m, n, k):
-    """Grids that take the bfloat16 split: magnitudes over 40 binades within the
-    bound of test_gemm_f32_tiles (the three parts are exact and the products
-    left out below 3 x 2^-24 of their magnitude), infinities and NaN as in fp32."""
+    """Grids that take the bfloat16 split (from K = 64 on): magnitudes over 40
+    binades within the bound of test_gemm_f32_tiles (the three parts are exact
+    and the products left out below 1.001 x 2^-24 of their magnitude),
+    infinities and NaN as in fp32."""
     torch = gpu
     _announce("gemm_f32 split", m, n, k)
     g = torch.Generator().manual_seed(m + n + k)
@@ -143,6 +144,67 @@ def test_gemm_f32_split(gpu, pkg, lib, m, n, k):
     assert torch.equal(out[~finite].nan_to_num(1.0, 2.0, 3.0).double(), want[~finite].nan_to_num(1.0, 2.0, 3.0))
     mag = ad.double().abs() @ bd.double().abs().T
     assert bool(((out.double() - want).abs()[finite] <= (2 * k + 3) * 2.0 ** -24 * mag[finite]).all())
+
+
+@pytest.mark.parametrize("family,k", [("one product", 64), ("one product", 1024), ("normal", 64), ("normal", 1028),
+                                      ("positive", 384), ("positive", 4096), ("tiny", 64), ("subnormal", 128)])
+def test_gemm_f32_split_precision(gpu, pkg, lib, family, k):
+    """The bfloat16 split against float64, in units of 2^-24 of the sum of
+    magnitudes: the products left out 1.001, the last addition 1, the small sums
+    2^-6, and every MFMA (32 k) up to 2 of the sum it ends with, a truncation.
+    Sums of positive products grow in proportion, so theirs average half the last
+    one; a sum of one product is exact up to the last addition."""
+    torch = gpu
+    _announce("gemm_f32 split precision", family, k)
+    m, n = 2001, 2100
+    g = torch.Generator().manual_seed(k)
+    a, b = torch.randn((m, k), generator=g), torch.randn((n, k), generator=g)
+    steps = (k + 31) // 32
+    bound = 2.02 + 2 * steps
+    if family == "one product":  # of mantissas whose left-out parts are largest, cut off or rounded
+        one = torch.zeros((m, k))
+        worst = torch.tensor([1 + 2.0 ** -7 - 2.0 ** -23, 1 + 2.0 ** -8 - 2.0 ** -17 - 2.0 ** -23])
+        row, col = torch.arange(m), torch.arange(n)
+        one[row, row % k] = torch.where(row % 3 == 2, a[:, 0], worst[row % 2])
+        a, b, bound = one, torch.where(col[:, None] % 3 == 2, b, worst[col % 2][:, None]), 2.02
+    elif family == "positive":
+        a, b, bound = a.abs(), b.abs(), 4.0 + steps
+    elif family in ("tiny", "subnormal"):
+        a, b = a * 2.0 ** (-120 if family == "tiny" else -130), b * 2.0 ** 100
+    ad, bd = a.cuda(), b.cuda()
+    out = torch.full((m, n), float("nan"), device="cuda")
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue, args.out = m, n, k, 1, ptr(out)
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    want = ad.double() @ bd.double().T
+    mag = ad.double().abs() @ bd.double().abs().T
+    assert bool(((out.double() - want).abs() <= bound * 2.0 ** -24 * mag).all())
+
+
+def test_gemm_f32_split_range(gpu, pkg, lib):
+    """Operands and sums past the split's range are summed in fp32, and only
+    those: the other sums keep their bits."""
+    torch = gpu
+    m, n, k = 2048, 2112, 96
+    g = torch.Generator().manual_seed(3)
+    ad, bd = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    args = pkg.GemmF32Args()
+    out = torch.full((2, m, n), float("nan"), device="cuda")
+    args.lda, args.b, args.ldb = k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue = m, n, k, 1
+    large = ad.clone()
+    large[::5] *= 2.0 ** 104  # past bfloat16 parts
+    large[1::5] *= 2.0 ** 90  # sums past the largest float once scaled
+    for i, x in enumerate((ad, large)):
+        args.a, args.out = ptr(x), ptr(out[i])
+        ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    want = large.double() @ bd.double().T
+    mag = large.double().abs() @ bd.double().abs().T
+    assert bool(((out[1].double() - want).abs() <= 2 * k * 2.0 ** -24 * mag).all())
+    rest = torch.ones(m, dtype=torch.bool, device="cuda")
+    rest[::5] = rest[1::5] = False
+    assert torch.equal(out[0][rest], out[1][rest])
 
 
 def test_gemm_f32_rejects(gpu, pkg, lib):
