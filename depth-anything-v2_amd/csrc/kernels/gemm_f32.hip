@@ -304,7 +304,7 @@ DAV2_DEV void split_bf16(v4f x, v2u (&part)[3]) {
 
 // fp32 operands on the bfloat16 MFMA: each operand is split into three parts
 // on its way into LDS (global -> registers, two stages ahead -> three planes of
-// 64-byte rows) and six products per element go to v_mfma_f32_16x16x32_bf16: 96
+// BK values a row) and six products per element go to v_mfma_f32_16x16x32_bf16: 96
 // matrix cycles for 32 k of a block where v_mfma_f32_16x16x4_f32 takes 256. The
 // three left out (parts 1 and 2, twice, and 2 and 2) are at most (1 + 2^-10)
 // 2^-24 of the element's product. Products of the same order (part numbers that
@@ -317,12 +317,12 @@ DAV2_DEV void split_bf16(v4f x, v2u (&part)[3]) {
 // left-out products 9.3e-8 / 2.1e-7 / 5.2e-7 / 8.8e-6 -> 6.2e-8 / 6.6e-8 / 6.2e-8 /
 // 6.8e-8. What bounds it: LDS (four plane reads and one write for each product of
 // a 32x32 wave block) and the VALU's splitting.
-template <int BN, int BM, int WN, int WM, int EPI>
+template <int BN, int BM, int WN, int WM, int BK, int EPI>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
     constexpr int NT = 64 * WN * WM, TN = BN / WN / 16, TM = BM / WM / 16;
-    constexpr int ROWS = BN + BM, LPT = ROWS * 8 / NT;  // float4 loads per thread and stage
-    constexpr int PLANE = ROWS * 64, STAGE = 3 * PLANE;  // bytes
-    static_assert(TN * WN * 16 == BN && TM * WM * 16 == BM && LPT * NT == ROWS * 8, "whole blocks and loads");
+    constexpr int ROWS = BN + BM, QK = BK / 4, LPT = (ROWS * QK + NT - 1) / NT;  // float4 loads per thread and stage
+    constexpr int PLANE = ROWS * BK * 2, STAGE = 3 * PLANE;  // bytes
+    static_assert(TN * WN * 16 == BN && TM * WM * 16 == BM && NT % QK == 0, "whole blocks and rows");
     extern __shared__ __attribute__((aligned(16))) int8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -331,30 +331,31 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
     uint32_t tm, tn;
     tile_of(tm, tn);
     const uint32_t row0 = tm * BM, col0 = tn * BN;
-    const int steps = static_cast<int>((g.k + kBK - 1) / kBK);
+    const int steps = static_cast<int>((g.k + BK - 1) / BK);
 
-    // Thread t's load i is float4 t % 8 of stage row t / 8 + i NT / 8. Rows
-    // past the matrix read its last row (never stored), k past K is zero.
-    const uint32_t kq = 4u * (tid & 7);
+    // Thread t's load i is float4 t % QK of stage row t / QK + i NT / QK (past
+    // the last row that one again, the same bytes). Rows past the matrix read
+    // its last row (never stored), k past K is zero.
+    const uint32_t kq = 4u * (tid % QK);
     const float* src[LPT];
     uint32_t dst[LPT];
 #pragma unroll
     for (int i = 0; i < LPT; ++i) {
-        const uint32_t r = (tid >> 3) + i * (NT / 8);
+        const uint32_t r = min(tid / QK + i * (NT / QK), ROWS - 1);
         src[i] = (r < static_cast<uint32_t>(BN) ? g.b + min(col0 + r, g.n - 1) * g.ldb
                                                 : g.a + min(row0 + r - BN, g.m - 1) * g.lda) + kq;
-        dst[i] = swz<64>(r, (tid & 7) >> 1) + 8u * (tid & 1);
+        dst[i] = swz<2 * BK>(r, (tid % QK) >> 1) + 8u * (tid & 1);
     }
     v4f next[2][LPT];
     auto load = [&](int step, auto set) {
-        const bool in = static_cast<uint32_t>(step) * kBK + kq < g.k;
+        const bool in = static_cast<uint32_t>(step) * BK + kq < g.k;
 #pragma unroll
         for (int i = 0; i < LPT; ++i) {
-            next[decltype(set)::value][i] = *reinterpret_cast<const v4f*>(src[i] + (in ? step * kBK : -static_cast<int>(kq)));
+            next[decltype(set)::value][i] = *reinterpret_cast<const v4f*>(src[i] + (in ? step * BK : -static_cast<int>(kq)));
         }
     };
     auto stash = [&](int step, auto set) {
-        const bool in = static_cast<uint32_t>(step) * kBK + kq < g.k;
+        const bool in = static_cast<uint32_t>(step) * BK + kq < g.k;
         int8_t* st = smem + decltype(set)::value * STAGE;
 #pragma unroll
         for (int i = 0; i < LPT; ++i) {
@@ -380,32 +381,40 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
     __syncthreads();
     auto stage = [&](int step, auto cur, auto nxt) {
         const int8_t* st = smem + decltype(cur)::value * STAGE;
-        v8b pf[3][TN], qf[3][TM];
+        v8b pf[BK / 32][3][TN], qf[BK / 32][3][TM];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
+        for (int h = 0; h < BK / 32; ++h)
 #pragma unroll
-            for (int i = 0; i < TN; ++i)
-                pf[k][i] = *reinterpret_cast<const v8b*>(st + k * PLANE + swz<64>(wn * (TN * 16) + i * 16 + fr, fg));
+            for (int k = 0; k < 3; ++k) {
+                const int8_t* plane = st + k * PLANE;
 #pragma unroll
-            for (int j = 0; j < TM; ++j)
-                qf[k][j] = *reinterpret_cast<const v8b*>(st + k * PLANE + swz<64>(BN + wm * (TM * 16) + j * 16 + fr, fg));
-        }
+                for (int i = 0; i < TN; ++i)
+                    pf[h][k][i] =
+                        *reinterpret_cast<const v8b*>(plane + swz<2 * BK>((wn * TN + i) * 16 + fr, 4 * h + fg));
+#pragma unroll
+                for (int j = 0; j < TM; ++j)
+                    qf[h][k][j] =
+                        *reinterpret_cast<const v8b*>(plane + swz<2 * BK>(BN + (wm * TM + j) * 16 + fr, 4 * h + fg));
+            }
         // unconditional (past the last stage it is loaded again and never
         // read), so that the waits count the other set's loads as in flight
         stash(step + 1, nxt);
         load(min(step + 3, steps - 1), nxt);
-        __builtin_amdgcn_sched_barrier(0);
         constexpr int pp[6] = {2, 1, 0, 1, 0, 0}, qq[6] = {0, 0, 0, 1, 1, 2};
 #pragma unroll
-        for (int t = 0; t < 6; ++t)
+        for (int h = 0; h < BK / 32; ++h)
 #pragma unroll
-            for (int i = 0; i < TN; ++i)
+            for (int t = 0; t < 6; ++t)
 #pragma unroll
-                for (int j = 0; j < TM; ++j) {
-                    const int order = pp[t] + qq[t];
-                    v4f& sum = order == 0 ? acc[i][j] : order == 1 ? mid[i][j] : low[i][j];
-                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[pp[t]][i], qf[qq[t]][j], sum, 0, 0, 0);
-                }
+                for (int i = 0; i < TN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TM; ++j) {
+                        const int order = pp[t] + qq[t];
+                        v4f& sum = order == 0 ? acc[i][j] : order == 1 ? mid[i][j] : low[i][j];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pf[h][pp[t]][i], qf[h][qq[t]][j], sum, 0, 0, 0);
+                    }
+        // this wave's reads of the stage and its writes of the next have
+        // ended; after the barrier every wave's have
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
     };
@@ -648,38 +657,68 @@ void launch_tiles(const F32Params& g, hipStream_t s) {
     }
 }
 
-// From 512 tiles of 128x64 on (two for every CU) the bfloat16 split of 128x64
-// on 8 waves: us against the best of the above at rows x N x K 1370 x 4096 x
-// 1024 with GELU 101 / 138, 1814 x 3072 x 768 72 / 98, 1814 x 2304 x 768 66 /
-// 73, 5480 x 3072 x 1024 256 / 330; below that it does not fill the chip (1814 x
-// 768 x 3072 93-98 / 93, 1370 x 1024 x 1024 40 / 38), nor do its 64x64 (32x32)
-// tiles beat the above (43, 49).
-//
-// Below K = 64 the products the split leaves out can cost more than the sums of
-// the fp32 MFMA: 6.2e-8 against 3.3e-8 / 6.1e-8 / 7.7e-8 / 9.3e-8 at K = 8 / 32 / 48
-// / 64 for operands chosen for it.
-constexpr uint32_t kSplitDepth = 64;
-
-template <int EPI>
-void launch_f32(const F32Params& g, hipStream_t s) {
-    constexpr uint32_t kBn = 128, kBm = 64;
-    constexpr size_t lds = 2u * 3u * (kBn + kBm) * 64u;
-    static const bool roomy =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<kBn, kBm, 4, 2, EPI>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) == hipSuccess;
-    if (roomy && g.k >= kSplitDepth && static_cast<uint64_t>(ceil_div(g.n, kBn)) * ceil_div(g.m, kBm) >= 2u * kCus)
-        dispatch(gemm_split_kernel<kBn, kBm, 4, 2, EPI>, dim3(ceil_div(g.m, kBm), ceil_div(g.n, kBn)), dim3(512), lds,
-                 s, g);
-    else
-        launch_tiles<false, EPI>(g, s);
+template <int BN, int BM, int WN, int WM, int BK, int EPI>
+void launch_split_tile(const F32Params& g, hipStream_t s) {
+    constexpr size_t lds = 2u * 3u * (BN + BM) * BK * 2u;
+    if (lds > 64u * 1024u) {
+        static const hipError_t attr =
+            hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<BN, BM, WN, WM, BK, EPI>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        (void)attr;
+    }
+    dispatch(gemm_split_kernel<BN, BM, WN, WM, BK, EPI>, dim3(ceil_div(g.m, BM), ceil_div(g.n, BN)),
+             dim3(64 * WN * WM), lds, s, g);
 }
+
+// The tile of the split changes no bits. The time of its grid: that of one tile
+// on a CU, and less for each further one on the busiest CU, by what they leave
+// each other (us at K = 1024, in the table below; 32x32 goes in stages of 64 k).
+// us by its order, then the best of launch_tiles<false>, which is ahead by up to a
+// tenth on the smallest grids only: 31 x 1024 x 1024 12.0 / 20 / 25 / 29, 11.4; 253 x
+// 1024 x 1024 13 / 21 / 26 / 30, 12; 253 x 768 x 3072 31 / 56 / 69 / 81, 30; 545 x
+// 3072 x 768 36 / 28 / 39 / 25, 33; 1370 x 768 x 768 27 / 27 / 22 / 25, 24; 1370 x
+// 768 x 3072 92 / 93 / 70 / 81, 79; 1370 x 1024 x 4096 150 / 130 / 178 / 109, 119;
+// 1370 x 4096 x 1024 148 / 106 / 130 / 87, 118; 5477 x 1024 x 4096 537 / 375 / 446 /
+// 319, 437. A sched_barrier between the splitting and the products cost 128x64 20%
+// (99 / 82 at 1370 x 4096 x 1024).
+template <int EPI>
+void launch_split(const F32Params& g, hipStream_t s) {
+    struct Tile {
+        uint32_t bn, bm;
+        double first, more;
+    };
+    constexpr Tile tiles[] = {{32, 32, 12.5, 5.5}, {64, 64, 21.5, 17.0}, {64, 80, 25.5, 24.5}, {128, 64, 30.5, 24.5}};
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        if (ceil_div(g.n, tiles[i].bn) > 65535u) continue;  // grid limit; f32_params checked it for 64 columns
+        const uint64_t count = static_cast<uint64_t>(ceil_div(g.n, tiles[i].bn)) * ceil_div(g.m, tiles[i].bm);
+        const double cost = tiles[i].first + tiles[i].more * static_cast<double>(ceil_div(count, kCus) - 1u);
+        if (best < 0 || cost < least) best = i, least = cost;
+    }
+    switch (best) {
+        case 0: launch_split_tile<32, 32, 2, 2, 64, EPI>(g, s); break;
+        case 1: launch_split_tile<64, 64, 4, 2, 32, EPI>(g, s); break;
+        case 2: launch_split_tile<64, 80, 2, 5, 32, EPI>(g, s); break;
+        default: launch_split_tile<128, 64, 4, 2, 32, EPI>(g, s); break;
+    }
+}
+
+// Which arithmetic sums a row depends on K alone, so that a row's bits do not
+// depend on the rows that come with it (an image's on its batch). Below K = 64
+// the products the split leaves out can cost more than the sums of the fp32
+// MFMA: 6.2e-8 against 3.3e-8 / 6.1e-8 / 7.7e-8 / 9.3e-8 at K = 8 / 32 / 48 / 64 for
+// operands chosen for it.
+constexpr uint32_t kSplitDepth = 64;
 
 template <int EPI>
 void launch(const F32Params& g, hipStream_t s) {
     if (g.half_operands)
         launch_tiles<true, EPI>(g, s);
+    else if (g.k < kSplitDepth)
+        launch_tiles<false, EPI>(g, s);
     else
-        launch_f32<EPI>(g, s);
+        launch_split<EPI>(g, s);
 }
 
 template <int EPI>

@@ -207,6 +207,30 @@ def test_gemm_f32_split_range(gpu, pkg, lib):
     assert torch.equal(out[0][rest], out[1][rest])
 
 
+@pytest.mark.parametrize("half", [0, 1])
+@pytest.mark.parametrize("n,k", [(384, 384), (772, 1028), (4096, 128), (1155, 44), (768, 64), (31, 60)])
+def test_gemm_f32_rows_alone(gpu, pkg, lib, n, k, half):
+    """A row's bits do not depend on the rows that come with it, whatever tile
+    or arithmetic the sizes choose; an infinite row leaves the others alone."""
+    torch = gpu
+    _announce("gemm_f32 rows", n, k, half)
+    g = torch.Generator().manual_seed(n + k)
+    m = 5481
+    ad, bd = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    ad[70, 1] = float("inf")
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.n, args.k, args.epilogue, args.half_operands = n, k, 1, half
+    whole = torch.full((m, n), float("nan"), device="cuda")
+    args.m, args.out = m, ptr(whole)
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    for rows in (1, 33, 70, 253, 545, 1370, 1814, 2740):
+        out = torch.full((rows, n), float("nan"), device="cuda")
+        args.m, args.out = rows, ptr(out)
+        ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+        assert torch.equal(out.view(torch.int32), whole[:rows].view(torch.int32)), rows
+
+
 def test_gemm_f32_rejects(gpu, pkg, lib):
     torch = gpu
     a = empty(torch, (8, 8), torch.float32)
@@ -397,3 +421,29 @@ def test_fp32_mode_depth_parity(gpu, pkg, lib, oracle, models, enc, width, heigh
     e_depth, e_logits = _span_err(depth, ref_depth), _span_err(logits, ref_logits)
     print(f"fp32 parity {enc} {width}x{height}: depth {e_depth:.3g}, logits {e_logits:.3g}", flush=True)
     assert e_depth <= 1e-3 and e_logits <= 1e-3
+
+
+@pytest.mark.parametrize("mode", ["FORCE_FP32", "FORCE_FP16"])
+def test_float_modes_batch_equals_singles(gpu, pkg, lib, tmp_path, mode):
+    """An image's depth has the same bits alone and in a batch of eight (3808 token
+    rows); LayerScale large enough for the blocks to reach the output, a head
+    whose depth varies."""
+    torch = gpu
+    _announce("float mode batch", mode)
+    width, height, batch = 350, 266, 8
+    state = pkg.dav2_format.synthetic_state("vits", SEED + 9)
+    path = tmp_path / "vits.dav2"
+    state = {k: v + 0.1 if k.endswith("gamma") else v for k, v in state.items()}
+    state["depth_head.scratch.output_conv2.2.weight"] = state["depth_head.scratch.output_conv2.2.weight"] * 8.0
+    state["depth_head.scratch.output_conv2.2.bias"] = state["depth_head.scratch.output_conv2.2.bias"] + 0.25
+    pkg.dav2_format.write_model(path, "vits", state)
+    xd = dev(torch, pkg.dav2_format.imagenet_input(width, height, seed=SEED + 5, batch=batch))
+    out, single = empty(torch, (batch, height, width), torch.float32), empty(torch, (height, width), torch.float32)
+    s = torch.cuda.current_stream().cuda_stream
+    with pkg.Context(str(path), "vits", getattr(pkg, mode)) as ctx:
+        ctx.infer_device(xd.data_ptr(), batch, width, height, out.data_ptr(), out.numel(), s)
+        together = host(torch, out)
+        assert together.std() > 1e-3
+        for b in range(batch):
+            ctx.infer_device(xd[b].data_ptr(), 1, width, height, single.data_ptr(), single.numel(), s)
+            assert np.array_equal(host(torch, single).view(np.uint32), together[b].view(np.uint32)), b
