@@ -207,6 +207,72 @@ def test_gemm_f32_split_range(gpu, pkg, lib):
     assert torch.equal(out[0][rest], out[1][rest])
 
 
+@pytest.mark.parametrize("w,h,n,k", [(31, 1, 63, 68), (109, 5, 1017, 132), (137, 10, 765, 64), (2081, 1, 2052, 100)])
+@pytest.mark.parametrize("epi", ["row", "gelu", "layerscale", "transposed", "convt"])
+def test_gemm_f32_split_epilogues(gpu, pkg, lib, oracle, w, h, n, k, epi):
+    """Every tile of the split with every epilogue, ragged: LayerScale in place,
+    an output offset, and an infinite row whose block is summed again."""
+    torch = gpu
+    _announce("gemm_f32 split epilogues", w, h, n, k, epi)
+    m = w * h
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+    bias, gamma = rng.standard_normal(n).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    v = a.astype(np.float64) @ b.astype(np.float64).T
+    a[7, 2] = np.inf
+    ad, bd, biasd, gd = dev(torch, a), dev(torch, b), dev(torch, bias), dev(torch, gamma)
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue, args.bias = m, n, k, EPI[epi], ptr(biasd)
+    if epi == "convt":
+        c = n // 9
+        out = empty(torch, (c, 3 * h, 3 * w), torch.float32)
+        args.convt_kernel, args.convt_width, args.convt_height, args.convt_channels = 3, w, h, c
+        want = v.reshape(h, w, 3, 3, c).transpose(4, 0, 2, 1, 3).reshape(c, 3 * h, 3 * w) + bias[:c, None, None]
+        row7 = np.zeros((h, w), bool)
+        row7.reshape(-1)[7] = True
+        row7 = np.broadcast_to(np.kron(row7, np.ones((3, 3), bool)), want.shape)
+    elif epi == "transposed":
+        res = rng.standard_normal((n, m + 5)).astype(np.float32)
+        out, resd = dev(torch, res), dev(torch, res)
+        args.out, args.out_row_stride, args.out_row_offset, args.residual = ptr(out), m + 5, 3, ptr(resd)
+        args.relu_output = 1
+        want = res.astype(np.float64)
+        want[:, 3:3 + m] = np.maximum(v.T + bias[:, None] + want[:, 3:3 + m], 0.0)
+        row7 = np.zeros(want.shape, bool)
+        row7[:, 10] = True
+    else:
+        res = rng.standard_normal((m + 1, n)).astype(np.float32)
+        out = dev(torch, res)
+        args.out_row_offset = 1
+        want = res.astype(np.float64)
+        if epi == "layerscale":
+            args.residual, args.gamma = ptr(out), ptr(gd)
+            want[1:] += (v + bias) * gamma
+        else:
+            want[1:] = oracle.gelu((v + bias).astype(np.float32)) if epi == "gelu" else v + bias
+        row7 = np.zeros(want.shape, bool)
+        row7[8] = True
+    args.out = ptr(out)
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    got = host(torch, out)
+    assert _rel(got[~row7], want[~row7]) < 1e-5
+    # the infinite row: +-inf by the weight's sign (GELU of -inf is NaN, ReLU of it 0)
+    sign = np.sign(b[:, 2])
+    if epi == "convt":
+        seven = got.reshape(c, h, 3, w, 3)[:, 7 // w, :, 7 % w, :].transpose(1, 2, 0).reshape(-1)
+        assert np.array_equal(seven, np.inf * sign)
+    elif epi == "transposed":
+        assert np.array_equal(got[:, 10], np.where(sign > 0, np.inf, 0.0))
+    elif epi == "layerscale":
+        assert np.array_equal(got[8], np.inf * sign * np.sign(gamma))
+    elif epi == "gelu":
+        assert np.all(got[8][sign > 0] == np.inf) and not np.any(np.isposinf(got[8][sign < 0]))
+    else:
+        assert np.array_equal(got[8], np.inf * sign)
+
+
 @pytest.mark.parametrize("half", [0, 1])
 @pytest.mark.parametrize("n,k", [(384, 384), (772, 1028), (4096, 128), (1155, 44), (768, 64), (31, 60)])
 def test_gemm_f32_rows_alone(gpu, pkg, lib, n, k, half):
@@ -423,6 +489,33 @@ def test_fp32_mode_depth_parity(gpu, pkg, lib, oracle, models, enc, width, heigh
     assert e_depth <= 1e-3 and e_logits <= 1e-3
 
 
+def _live_model(pkg, path, encoder, seed):
+    """A model whose blocks reach its output: LayerScale 0.1 and a head whose depth varies."""
+    state = pkg.dav2_format.synthetic_state(encoder, seed)
+    state = {k: v + 0.1 if k.endswith("gamma") else v for k, v in state.items()}
+    state["depth_head.scratch.output_conv2.2.weight"] = state["depth_head.scratch.output_conv2.2.weight"] * 8.0
+    state["depth_head.scratch.output_conv2.2.bias"] = state["depth_head.scratch.output_conv2.2.bias"] + 0.25
+    pkg.dav2_format.write_model(path, encoder, state)
+    return path
+
+
+@pytest.mark.parametrize("enc,width,height", [("vits", 266, 182), ("vitb", 126, 154), ("vitl", 112, 98)])
+def test_fp32_mode_live_blocks_parity(gpu, pkg, lib, oracle, tmp_path, enc, width, height):
+    _announce("fp32 model, live blocks", enc, width, height)
+    path = _live_model(pkg, tmp_path / "model.dav2", enc, SEED + 9)
+    x = pkg.dav2_format.imagenet_input(width, height, seed=SEED + 2)[0]
+    with pkg.Context(str(path), enc, pkg.FORCE_FP32) as ctx:
+        depth = ctx.infer(x, width, height)
+    h = oracle.load_model(path, ENC[enc])
+    try:
+        ref, _ = oracle.infer_fp32(h, x, width, height)
+    finally:
+        oracle.free_model(h)
+    span, err = float(ref.max() - ref.min()), _span_err(depth, ref)
+    print(f"fp32 parity {enc} {width}x{height}: depth {err:.3g} of {span:.3g}", flush=True)
+    assert span > 1e-3 and err <= 1e-3
+
+
 @pytest.mark.parametrize("mode", ["FORCE_FP32", "FORCE_FP16"])
 def test_float_modes_batch_equals_singles(gpu, pkg, lib, tmp_path, mode):
     """An image's depth has the same bits alone and in a batch of eight (3808 token
@@ -431,12 +524,7 @@ def test_float_modes_batch_equals_singles(gpu, pkg, lib, tmp_path, mode):
     torch = gpu
     _announce("float mode batch", mode)
     width, height, batch = 350, 266, 8
-    state = pkg.dav2_format.synthetic_state("vits", SEED + 9)
-    path = tmp_path / "vits.dav2"
-    state = {k: v + 0.1 if k.endswith("gamma") else v for k, v in state.items()}
-    state["depth_head.scratch.output_conv2.2.weight"] = state["depth_head.scratch.output_conv2.2.weight"] * 8.0
-    state["depth_head.scratch.output_conv2.2.bias"] = state["depth_head.scratch.output_conv2.2.bias"] + 0.25
-    pkg.dav2_format.write_model(path, "vits", state)
+    path = _live_model(pkg, tmp_path / "vits.dav2", "vits", SEED + 9)
     xd = dev(torch, pkg.dav2_format.imagenet_input(width, height, seed=SEED + 5, batch=batch))
     out, single = empty(torch, (batch, height, width), torch.float32), empty(torch, (height, width), torch.float32)
     s = torch.cuda.current_stream().cuda_stream
