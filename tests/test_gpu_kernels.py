@@ -805,6 +805,21 @@ def test_attention_f32_fused(gpu, lib, tokens, heads, batch, sigma):
     assert lib.dav2_hip_attention_f32(0, ptr(qd), tokens, heads, batch, stream(torch)) != 0
 
 
+@pytest.mark.parametrize("tokens", [1, 2, 33, 1025, 1370])
+def test_attention_f32_fused_large_values(gpu, lib, tokens):
+    # values near the largest float: their weighted mean is no larger
+    torch = gpu
+    _announce("fused fp32 attention, large values", tokens)
+    qkv = np.random.default_rng(tokens).standard_normal((tokens, 192)).astype(np.float32)
+    value = (np.linspace(-1.0, 1.0, 64) * 3.0e38).astype(np.float32)
+    qkv[:, 128:] = value
+    out = empty(torch, (tokens, 64), torch.float32)
+    ok(lib, lib.dav2_hip_attention_f32(ptr(out), ptr(dev(torch, qkv)), tokens, 1, 1, stream(torch)))
+    # numerator and denominator sum the same weights: a rounding for each of 32 keys a step and the division
+    bound = (tokens / 32 + 8) * 2.0 ** -23 * np.abs(value.astype(np.float64))
+    assert np.all(np.abs(host(torch, out).astype(np.float64) - value) <= bound)
+
+
 @pytest.mark.parametrize("tokens,heads,batch", [(1, 1, 1), (5, 2, 1), (65, 3, 1), (258, 2, 2), (1370, 6, 1),
                                                 (1370, 16, 1)])
 def test_attention_ref_fp32_bit_exact(gpu, lib, oracle, tokens, heads, batch):
