@@ -17,11 +17,12 @@
 //
 // Bound: the fp32 MFMA (157 TFLOP/s). No im2col matrix is written and read
 // back (9 times the input: 101 MB each way for 148x148x128), which took half
-// to two thirds of the time of im2col + GEMM. us, im2col + GEMM -> this: 148x148
-// 128 -> 128 159 -> 78 (83 TFLOP/s), 74x74 128 -> 128 46 -> 27, 296x296 128 ->
-// 64 509 -> 141 (92), 518x518 64 -> 32 693 -> 120 (82), 37x37 1024 -> 256 170
-// -> 127; 1x1 296x296 128 -> 128 98 -> 43. Three or four slots measured the
-// same as two; reading each step's operands where they are used, 5% slower.
+// to two thirds of the time of im2col + GEMM. us, im2col + GEMM (which
+// reads the matrix on the bfloat16 split) / this: 148x148 128 -> 128 129 / 70 (93
+// TFLOP/s), 74x74 128 -> 128 45 / 25, 296x296 128 -> 64 458 / 130 (99), 518x518 64
+// -> 32 684 / 103 (96), 37x37 1024 -> 256 154 / 124; 1x1 296x296 128 -> 128 92 / 44.
+// Three or four slots measured the same as two; reading each step's operands
+// where they are used, 5% slower.
 
 #include <type_traits>
 
@@ -149,8 +150,12 @@ __global__ __launch_bounds__(256) void conv_f32_kernel(ConvF32Params g) {
     auto walk = [&](auto relu) {
         issue(0);
         for (int s = 0; s < stages; ++s) {
-            DAV2_WAIT_VMCNT(0);            // this wave's copies of the stage
-            __builtin_amdgcn_s_barrier();  // everyone's; the operands of the other slot have been used
+            // this wave's copies of the stage have landed and its reads of the
+            // other slot have ended (vmcnt(0) lgkmcnt(0)); after the barrier every
+            // wave's have, and the other slot is free
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0x0070);
+            __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
             if (s + 1 < stages) issue(s + 1);
             const float* w = lds[s & 1] + (wn * (TN * 16) + fr) * ROW + fg * TAPS;
