@@ -595,16 +595,20 @@ void HipOperators::conv2d(DeviceBuffer& output, const DeviceBuffer& input, const
     if (fusion.residual) require_bytes(*fusion.residual, pixels * output_channels, "convolution residual");
     const hipStream_t s = stream();
     // Implicit GEMM, unless the map is small and the channels are many: a few
-    // workgroups then walk all of them one after the other, and the 16-k steps
-    // of the GEMM are the shorter chain (19x19, 768 -> 128: 72 us for im2col +
-    // GEMM, 78 implicit; 37x37, 1024 -> 256: 170 and 127). The output may be
-    // the input's own buffer, which im2col has read before the GEMM writes.
+    // workgroups then walk all of them one after the other, and the 64-k steps
+    // of the GEMM are the shorter chain. us, implicit / im2col + GEMM, 3x3: 13x13
+    // 256 -> 128 25 / 28, 384 -> 64 36 / 40, 512 -> 256 48 / 52, 768 -> 128 70 / 76,
+    // 1024 -> 256 109 / 98; 30x30 256 -> 128 25 / 38, 384 -> 64 36 / 51, 1024 -> 256
+    // 107 / 118; 37x37 1024 -> 256 123 / 156. 1x1: 19x19 256 -> 128 7.4 / 8.1, 384 ->
+    // 64 9.8 / 9.7, 512 -> 256 12.5 / 11.6, 1024 -> 256 22 / 18; 37x37 1024 -> 256 28 /
+    // 28. The output may be the input's own buffer, which im2col has read before
+    // the GEMM writes.
     const auto at = [](const DeviceBuffer& b) { return reinterpret_cast<std::uintptr_t>(b.data()); };
     const bool overlaps = at(output) < at(input) + std::uint64_t(input_width) * input_height * input_channels * 4u &&
                           at(input) < at(output) + pixels * output_channels * 4u;
     if (dav2_hip_conv2d_f32_supported(input_width, input_height, input_channels, output_channels, kernel, stride,
                                       padding) &&
-        !overlaps && at(weight) % 16u == 0 && (pixels >= 1024u || input_channels <= 128u)) {
+        !overlaps && at(weight) % 16u == 0 && (pixels >= 1024u || input_channels <= 384u)) {
         dav2_conv_f32_args a{};
         a.input = input.as<float>();
         a.width = input_width;

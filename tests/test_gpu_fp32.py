@@ -387,6 +387,12 @@ def test_conv2d_f32_implicit(gpu, pkg, lib, c, oc, h, w, k, fused):
     assert bool(((out.double().cpu() - want).abs() <= (2 * c * k * k + 2) * 2.0 ** -24 * mag).all())
 
 
+@pytest.mark.parametrize("c,h,w", [(384, 7, 9), (400, 7, 9), (400, 32, 32)])
+def test_ops_conv2d_routes(gpu, pkg, lib, oracle, ops, c, h, w):
+    """Both sides of the line between the implicit GEMM and im2col, 1024 pixels and 384 channels."""
+    test_ops_conv2d(gpu, pkg, lib, oracle, ops, c, 40, h, w, 3, 1, 1)
+
+
 def test_ops_conv2d_in_place(gpu, pkg, lib, ops):
     """The output may be the input's buffer (im2col has read it before the GEMM writes)."""
     torch = gpu
