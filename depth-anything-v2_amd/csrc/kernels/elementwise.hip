@@ -131,22 +131,23 @@ __global__ __launch_bounds__(kBlock) void bilinear_kernel(float* __restrict__ ou
 }
 
 // Upsampling (oh >= ih): a wave walks kStripRows output rows of 64 columns and
-// 8 channels and keeps the two horizontally blended source rows between them, so
-// that a source value is loaded once or twice (each output of bilinear_kernel
-// loads four), the next source row's loads in flight; the same operations on the
-// same values. The four waves take neighbouring tiles, or with maxima (channels %
-// 32 == 0) the 32 channels of one, and then write max |out| of them. Workgroups
-// are numbered so that each XCD takes a contiguous run of the map: neighbouring
-// row pieces, which share cache lines, meet in one L2.
+// 8 channels and keeps the two horizontally blended source rows between them,
+// the next source row's loads in flight: 2 - 2.5 loads per output at twice the
+// size where bilinear_kernel has 4; the same operations on the same values.
+// EXACT: no loads of a row that the strip does not use. The four waves take
+// neighbouring tiles, or with maxima (channels % 32 == 0) the 32 channels of one,
+// and then write max |out| of them. Workgroups are numbered so that each XCD
+// takes a contiguous run of the map: neighbouring row pieces, which share cache
+// lines, meet in one L2.
 //
-// Bound by the stores to memory (3 TB/s with the reads; the stores are scattered
-// over 8 planes). us on buffers out of the caches, bilinear_kernel -> this: 296 ->
-// 518, 128 channels 61.5 -> 57.7, with maxima 68.9 -> 61.2; 148 -> 296, 256 channels
-// 40.8 -> 37.0, with maxima 45.2 -> 39.1. Strips of 8 or 16 rows: the same on large
-// maps, 1-5 us slower on small ones; nontemporal stores 60-68.
+// Bound by the stores to memory (3.2 TB/s with the reads; the stores are
+// scattered over 8 planes). us on buffers out of the caches, bilinear_kernel ->
+// this: 296 -> 518, 128 channels 61.5 -> 52.3, with maxima 68.9 -> 54.4; 148 -> 296,
+// 256 channels 40.8 -> 34.0, with maxima 45.2 -> 35.8. Strips of 8 or 16 rows: the
+// same on large maps, 1-5 us slower on small ones; nontemporal stores 60-68.
 constexpr uint32_t kStripRows = 4;
 
-template <bool MAX>
+template <bool MAX, bool EXACT>
 __global__ __launch_bounds__(kBlock) void bilinear_up_kernel(float* __restrict__ out, const float* __restrict__ in,
                                                              uint32_t iw, uint32_t ih, uint32_t ow, uint32_t oh,
                                                              uint32_t channels, uint32_t tiles_x, uint32_t tiles_y,
@@ -193,12 +194,13 @@ __global__ __launch_bounds__(kBlock) void bilinear_up_kernel(float* __restrict__
             for (uint32_t k = 0; k < C; ++k) row[k] = a[k] * (1.0f - fx) + b[k] * fx;
         };
         float fy;
+        const uint32_t last = EXACT ? source_row(min(oy0 + kStripRows, oh) - 1u, fy) + 1u : 0u;  // the strip ends with
         uint32_t y = source_row(oy0, fy);
         load(y);
         blend(top);
         load(y + 1u);
         blend(bottom);
-        load(y + 2u);
+        if (!EXACT || y + 2u <= last) load(y + 2u);
         float* dst = out + static_cast<uint64_t>(c0) * oplane + static_cast<uint64_t>(oy0) * ow + ox;
 #pragma unroll
         for (uint32_t j = 0; j < kStripRows; ++j) {
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(kBlock) void bilinear_up_kernel(float* __restrict__
                 for (uint32_t k = 0; k < C; ++k) top[k] = bottom[k];
                 blend(bottom);
                 ++y;
-                load(y + 2u);
+                if (!EXACT || y + 2u <= last) load(y + 2u);
             }
             float m = 0.0f;
 #pragma unroll
@@ -235,6 +237,10 @@ __global__ __launch_bounds__(kBlock) void bilinear_up_kernel(float* __restrict__
 // at 37 -> 74, 256 channels 5.1 / 5.4, 74 -> 148 10.0 / 8.6); with the maxima this
 // one is faster from there too (6.5 / 5.4, 11.3 / 8.8), its waves sharing the 32
 // channels. Fewer output rows than input rows would load rows no output needs.
+// EXACT from 8 Mi outputs, where the stores bound it; below, the branch delays
+// more than the loads cost (us, every row / EXACT: 296 -> 518, 128 channels, 34 M
+// 57.7 / 52.3, 64 channels, 17 M 29.4 / 27.7; 148 -> 296, 128, 11 M 18.9 / 16.9, 64,
+// 5.6 M 7.4 / 8.0; 74 -> 148, 256, 5.6 M 8.0 / 8.5).
 template <bool MAX>
 bool launch_bilinear_up(float* out, float* partial, const float* input, uint32_t iw, uint32_t ih, uint32_t ow,
                         uint32_t oh, uint32_t channels, hipStream_t s) {
@@ -243,8 +249,9 @@ bool launch_bilinear_up(float* out, float* partial, const float* input, uint32_t
     const uint64_t groups = MAX ? tiles * (channels / 32u) : (tiles + 3u) / 4u * ceil_div(channels, 8);
     if (oh < ih || groups > 0xffffffu) return false;
     if (!MAX && static_cast<uint64_t>(ow) * oh * channels < (4u << 20)) return false;
-    dispatch(bilinear_up_kernel<MAX>, dim3(static_cast<uint32_t>(groups)), dim3(kBlock), 0, s, out, input, iw, ih, ow,
-             oh, channels, tx, ty, partial);
+    const bool exact = static_cast<uint64_t>(ow) * oh * channels >= (8u << 20);
+    dispatch(exact ? bilinear_up_kernel<MAX, true> : bilinear_up_kernel<MAX, false>, dim3(static_cast<uint32_t>(groups)),
+             dim3(kBlock), 0, s, out, input, iw, ih, ow, oh, channels, tx, ty, partial);
     return true;
 }
 

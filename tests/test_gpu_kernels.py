@@ -1331,6 +1331,18 @@ def test_bilinear_strips_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow):
     test_bilinear_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow)
 
 
+@pytest.mark.parametrize("c,ih,iw,oh,ow", [(26, 201, 300, 599, 601), (70, 130, 350, 130, 950), (140, 1, 9, 241, 259),
+                                           (130, 127, 3, 1001, 65)])
+def test_bilinear_exact_strips_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow):
+    # from 8 Mi outputs on: the same edges, no row loaded past the strip's last
+    test_bilinear_bit_exact(gpu, lib, oracle, c, ih, iw, oh, ow)
+
+
+@pytest.mark.parametrize("c,ih,iw,oh,ow", [(32, 201, 300, 599, 601), (64, 400, 129, 401, 353)])
+def test_bilinear_maxima_exact_strips(gpu, lib, c, ih, iw, oh, ow):
+    test_bilinear_maxima(gpu, lib, c, ih, iw, oh, ow)
+
+
 @pytest.mark.parametrize("n", [4, 1000, 518 * 518, 1036 * 1036 + 5])
 def test_minmax_normalize(gpu, lib, oracle, n):
     torch = gpu
