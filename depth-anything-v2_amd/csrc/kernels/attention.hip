@@ -254,9 +254,9 @@ __global__ __launch_bounds__(256) void attention_values_kernel(const float* __re
 // Softmax online, in fp32: running maximum per query, the sums rescaled only
 // where a maximum grew, p = exp(s - max) / 2^s by expf; the division comes last.
 // Bounded by the fp32 MFMA (157 TFLOP/s). ViT-B 686x518 (T = 1814, 12
-// heads, 10.1 GFLOP): 523 us as scores + softmax + values (372 of them the
-// values) -> 128 us (79 TFLOP/s); 1370 tokens, 16 heads 374 -> 100; 5477 tokens,
-// 16 heads 3856 -> 1263 (99 TFLOP/s). Relative error against 64 bits 7.5e-7
+// heads, 10.1 GFLOP): 495 us as scores + softmax + values (365 of them the
+// values) -> 134 us (76 TFLOP/s); 1370 tokens, 16 heads 372 -> 103; 5477 tokens,
+// 16 heads 3857 -> 1259 (98 TFLOP/s). Relative error against 64 bits 7.5e-7
 // where the three kernels had 9.2e-7 (T = 1814).
 constexpr uint32_t kFlashRows = 32, kFlashKeys = 32;
 constexpr int kFlashSlot = kFlashKeys * 256;  // bytes

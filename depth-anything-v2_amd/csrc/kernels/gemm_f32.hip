@@ -725,8 +725,13 @@ template <int EPI>
 void launch_h16p(const F32Params& g, hipStream_t s) {
     const uint32_t nt = ceil_div(g.n, 32);
     const dim3 cols(0, min(nt, kMaxGridY), ceil_div(nt, kMaxGridY));
-    // two rows a thread halve the LDS reads of a product, one row gives twice
-    // the waves: us at 5476 x 1024 x 1024 331 / 354, 1369 x 768 x 768 74 / 66
+    // Two rows a thread halve the LDS reads of a product, one row gives twice
+    // the waves. us, two / one, by 64x32 tiles: 66 (1369 x 96 x 768) 34 / 20, 264
+    // (1369 x 384 x 768) 49 / 40, 528 (1369 x 768 x 768) 68 / 60; between 696 and
+    // 2080 within 6% either way by how the last round of workgroups falls (704,
+    // 1369 x 1024 x 768, 68 / 70; 1032, 2738 x 768 x 768, 105 / 100; 1760, 3480 x
+    // 1024 x 768, 145 / 152; 2064, 5476 x 768 x 768, 181 / 182); 2752 (5476 x 1024 x
+    // 768) 220 / 232
     if (static_cast<uint64_t>(ceil_div(g.m, 64)) * nt >= 8u * kCus)
         dispatch(gemm_h16p_kernel<2, EPI>, dim3(ceil_div(g.m, 64), cols.y, cols.z), dim3(256), 0, s, g);
     else

@@ -604,27 +604,31 @@ constexpr uint32_t kWideTileRows = 4096;
 // Columns of Q from which those GEMMs take 128x128 tiles on eight waves.
 constexpr uint32_t kWideTileCols = 3072;
 
-// Rows of P per tile of the configuration launch_epi picks, for the epilogue
-// with column maxima (the others take 32 in few_tiles grids): 128 / 64 for the
-// 128x128 / 64x128 tiles of the large row-major GEMMs without column maxima
-// (rows_p >= kWideTileRows), else 32, 96 or 64 as in the switch below.
 // Columns of Q from which the smaller row-major GEMMs without column maxima
 // (fc1 at batch 1) take 128x64 tiles on eight waves.
 constexpr uint32_t kTallTileCols = 4096;
 
 // Grids of at most one 64x64 tile a CU leave most of the chip idle while a
 // few waves walk K: 32x32 tiles on four waves (the column maxima, whose row
-// tiles the caller has counted, keep 64x64 and take eight waves). us at rows x N x K, 64x64 -> 32x32: 253 x 384 x 384
-// LayerScale 4.2 -> 3.3, 253 x 384 x 1536 7.8 -> 7.0, 253 x 1536 x 384 GELU 6.3 ->
-// 4.1, 252 x 384 x 384 channel-major 5.6 -> 3.7, 61 x 1024 x 4096 15.4 -> 11.9,
-// 545 x 768 x 768 (108 tiles) 5.7 -> 4.8, 1370 x 384 x 1536 (132) 8.0 -> 7.2; 1370
-// x 768 x 3072 (264) 15.7 -> 15.9, 1370 x 1024 x 1024 (352) 8.1 -> 8.7. Eight
-// waves: 253 x 1152 x 384 5.0 -> 4.1. Six stages in place of three: 0.2-0.5
+// tiles the caller has counted, keep 64x64 and take eight waves). us at rows x
+// N x K, 64x64 / 32x32: 253 x 384 x 384 LayerScale 4.2 / 3.3, 253 x 384 x 1536 7.8
+// / 7.0, 253 x 1536 x 384 GELU 6.3 / 4.1, 252 x 384 x 384 channel-major 5.6 / 3.7,
+// 61 x 1024 x 4096 15.4 / 11.9. By 64x64 tiles, N x K as named, without an
+// epilogue: 108 tiles (545 x 768 x 768) 5.3 / 4.5, 156 (784 x 768 x 3072) 12.7 /
+// 11.7, 208 (1024 x 832) K = 768 5.5 / 5.5, K = 4096 16.1 / 15.5, 256 (1024 x 1024)
+// 5.6 / 5.5 and 16.1 / 15.8, 272 (1025 x 1024) 6.2 / 6.0 and 17.5 / 17.9, 286 (1370
+// x 832) 6.3 / 6.1 and 17.8 / 18.8, 330 (1370 x 960) 6.4 / 6.6 and 18.6 / 22.5.
+// Eight waves: 253 x 1152 x 384 5.0 -> 4.1. Six stages in place of three: 0.2-0.5
 // slower but for the longest K.
 inline bool few_tiles(uint32_t rows_p, uint32_t rows_q, uint32_t slices) {
     return static_cast<uint64_t>(ceil_div(rows_p, 64)) * ceil_div(rows_q, 64) * slices <= 256u;
 }
 
+// Rows of P per tile of the configuration launch_epi picks outside few_tiles
+// grids, and within them for the epilogue with column maxima: 128 / 64 for the
+// 128x128 / 64x128 tiles of the large row-major GEMMs without column maxima
+// (rows_p >= kWideTileRows), 128 for the 128x64 ones, else 32, 96 or 64 as in
+// launch_epi's switch.
 inline uint32_t tile_rows(uint32_t rows_p, uint32_t rows_q, bool row_major, bool col_max) {
     if (row_major && !col_max && rows_p >= kWideTileRows) return rows_q >= kWideTileCols ? 128 : 64;
     if (row_major && !col_max && rows_q >= kTallTileCols && rows_p >= 512) return 128;
