@@ -1,10 +1,10 @@
 // Head-64 fp32 attention on the matrix cores, for the fp32 precision mode
 // (FORCE_FP32): softmax((0.125 q) k^T) v on v_mfma_f32_16x16x4_f32, fused
-// (flash_f32_kernel, the model's path), or as three launchers over
-// materialised scores. fp32 products and sums, in the matrix core's order, so
-// within tolerance of the reference (src/operators.cpp:1169-1208, bmm.glsl,
-// softmax_lastdim.glsl), not bit for bit; the reference-order kernels are in
-// attention_ref.hip.
+// (flash_f32_kernel, the model's path), or as three public launchers over
+// materialised scores, which no mode uses. fp32 products and sums, in the
+// matrix core's order, so within tolerance of the reference
+// (src/operators.cpp:1169-1208, bmm.glsl, softmax_lastdim.glsl), not bit for
+// bit; the reference-order kernels are in attention_ref.hip.
 //
 // Layouts: qkv [batch*T][3*H*64]; scores [batch][H][T][T].
 

@@ -182,9 +182,12 @@ typedef struct dav2_gemm_f32_args {
     const float* gamma;
     uint32_t convt_kernel, convt_width, convt_height, convt_channels;
     uint32_t relu_output;   /* TRANSPOSED only                                 */
-    /* 1: both operands rounded to binary16 before the (exact) products, fp32
-     * accumulation: the fp16 mode's cooperative-matrix linears
-     * (linear_coop_fp16.glsl, src/operators.cpp:540-768). 0: fp32. */
+    /* 1: both operands rounded to binary16 before the products, which are
+     * exact (subnormal operands too), fp32 accumulation: the fp16 mode's
+     * cooperative-matrix linears (linear_coop_fp16.glsl,
+     * src/operators.cpp:540-768). 0: fp32; from k = 64 on every product is
+     * within 1.001 x 2^-24 of itself before it is summed. An output's bits
+     * depend on its row of a and of b and on k alone, not on m or n. */
     uint32_t half_operands;
 } dav2_gemm_f32_args;
 DAV2_API int dav2_hip_gemm_f32(const dav2_gemm_f32_args* args, void* stream);
@@ -320,7 +323,9 @@ DAV2_API int dav2_hip_round_half(float* data, uint64_t count, void* stream);
 DAV2_API int dav2_hip_attention_f32(float* out, const float* qkv, uint32_t tokens, uint32_t heads,
                                     uint32_t batch, void* stream);
 
-/* fp32 attention, head_dim 64, on the matrix cores over materialised scores
+/* fp32 attention, head_dim 64, on the matrix cores over materialised scores,
+ * for callers that want scores or probabilities; no precision mode uses these
+ * (dav2_hip_attention_f32 is 3 to 4 times as fast)
  * (src/operators.cpp:1169-1208 with bmm.glsl and
  * softmax_lastdim.glsl, sums in the MFMA's order: within tolerance of the
  * reference, not bit for bit). qkv is [batch*T][3*H*64] token-major (q | k |

@@ -719,7 +719,8 @@ def test_pad_rows_i8(gpu, lib, rows, cols, ld):
 # ---------------------------------------------------------------------------
 # attention: scores -> softmax -> values
 def _attention_mfma_gpu(torch, lib, qkv, tokens, heads):
-    """fp32 attention on the matrix cores (the fp32 precision mode's path)."""
+    """fp32 attention on the matrix cores over materialised scores (the three public
+    launchers; the fp32 precision mode runs dav2_hip_attention_f32)."""
     qd = dev(torch, qkv)
     nbytes = lib.dav2_hip_attention_scratch_bytes(tokens, heads, 1, 0)
     buf = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
@@ -1042,6 +1043,21 @@ def test_attention_mfma_fp32(gpu, lib, oracle, tokens, heads):
     out, p = _attention_mfma_gpu(torch, lib, qkv, tokens, heads)
     np.testing.assert_allclose(p, p_ref, rtol=2e-5, atol=2e-7)
     np.testing.assert_allclose(out, ref, rtol=1e-4, atol=2e-6)
+
+
+def test_attention_f32_fused_kat(gpu, lib):
+    # tests/vulkan_smoke.cpp:540-628 through the fused kernel of the fp32 mode:
+    # within 2e-6 of the closed form
+    torch = gpu
+    tokens, heads = 5, 2
+    qkv = ((np.arange(tokens * 384) % 29 - 14) * 0.0078125).astype(np.float32).reshape(tokens, 384)
+    x = qkv.astype(np.float64).reshape(tokens, 3, heads, 64)
+    out = empty(torch, (tokens, heads * 64), torch.float32)
+    ok(lib, lib.dav2_hip_attention_f32(ptr(out), ptr(dev(torch, qkv)), tokens, heads, 1, stream(torch)))
+    for h in range(heads):
+        p = np.exp((x[:, 0, h] * 0.125) @ x[:, 1, h].T)
+        want = p @ x[:, 2, h] / p.sum(axis=1, keepdims=True)
+        assert np.abs(host(torch, out)[:, 64 * h:64 * h + 64] - want).max() <= 2e-6
 
 
 def test_attention_reference_kat(gpu, lib):
