@@ -132,6 +132,18 @@ DAV2_DEV bool vector_rows(const F32Params& g) {
     return g.n % 4u == 0 && (any & 15u) == 0;
 }
 
+// First row and column of this workgroup's tile; false past the last row. Row
+// tiles go to grid x, and on to z beyond kMaxRowTiles.
+template <int BN, int BM>
+DAV2_DEV bool tile_start(const F32Params& g, uint32_t& row0, uint32_t& col0) {
+    uint32_t tm, tn;
+    tile_of(tm, tn);
+    const uint64_t row = (static_cast<uint64_t>(blockIdx.z) * gridDim.x + tm) * BM;
+    row0 = static_cast<uint32_t>(row);
+    col0 = tn * BN;
+    return row < g.m;
+}
+
 // BN weight rows (operand P of the MFMA, whose four result registers are then
 // consecutive output columns) x BM activation rows per workgroup, WN x WM
 // waves.
@@ -146,9 +158,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_kernel(F32Params g) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave / WM, wm = wave % WM;
-    uint32_t tm, tn;
-    tile_of(tm, tn);
-    const uint32_t row0 = tm * BM, col0 = tn * BN;
+    uint32_t row0, col0;
+    if (!tile_start<BN, BM>(g, row0, col0)) return;
     const int steps = static_cast<int>((g.k + kBK - 1) / kBK);
 
     // Copy c brings stage rows 8 c .. + 7, lane l row + l / 8 and the 16-byte
@@ -328,9 +339,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_split_kernel(F32Params g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave / WM, wm = wave % WM;
     const int fr = lane & 15, fg = lane >> 4;
-    uint32_t tm, tn;
-    tile_of(tm, tn);
-    const uint32_t row0 = tm * BM, col0 = tn * BN;
+    uint32_t row0, col0;
+    if (!tile_start<BN, BM>(g, row0, col0)) return;
     const int steps = static_cast<int>((g.k + BK - 1) / BK);
 
     // Thread t's load i is float4 t % QK of stage row t / QK + i NT / QK (past
@@ -615,12 +625,20 @@ __global__ __launch_bounds__(256) void im2col_f32_kernel(const float* __restrict
     out[i] = v;
 }
 
+// A launch holds fewer than 2^32 threads in x; the tiles have at most 640.
+constexpr uint32_t kMaxRowTiles = 1u << 22;
+
+template <int BN, int BM>
+dim3 tile_grid(const F32Params& g) {
+    const uint32_t rows = ceil_div(g.m, BM), x = min(rows, kMaxRowTiles);
+    return dim3(x, ceil_div(g.n, BN), ceil_div(rows, x));
+}
+
 template <int BN, int BM, int WN, int WM, int STAGES, bool HALF, int EPI>
 void launch_tile(const F32Params& g, hipStream_t s) {
     constexpr size_t lds = static_cast<size_t>(STAGES) * (BN + BM) * 128u;
     static_assert(lds <= 64u * 1024u, "no larger dynamic LDS is asked for");
-    dispatch(gemm_f32_kernel<BN, BM, WN, WM, STAGES, HALF, EPI>, dim3(ceil_div(g.m, BM), ceil_div(g.n, BN)),
-             dim3(64 * WN * WM), lds, s, g);
+    dispatch(gemm_f32_kernel<BN, BM, WN, WM, STAGES, HALF, EPI>, tile_grid<BN, BM>(g), dim3(64 * WN * WM), lds, s, g);
 }
 
 constexpr uint32_t kCus = 256;  // MI355X
@@ -660,20 +678,19 @@ void launch_tiles(const F32Params& g, hipStream_t s) {
 template <int BN, int BM, int WN, int WM, int BK, int EPI>
 void launch_split_tile(const F32Params& g, hipStream_t s) {
     constexpr size_t lds = 2u * 3u * (BN + BM) * BK * 2u;
-    if (lds > 64u * 1024u) {
+    if constexpr (lds > 64u * 1024u) {
         static const hipError_t attr =
             hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_split_kernel<BN, BM, WN, WM, BK, EPI>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         (void)attr;
     }
-    dispatch(gemm_split_kernel<BN, BM, WN, WM, BK, EPI>, dim3(ceil_div(g.m, BM), ceil_div(g.n, BN)),
-             dim3(64 * WN * WM), lds, s, g);
+    dispatch(gemm_split_kernel<BN, BM, WN, WM, BK, EPI>, tile_grid<BN, BM>(g), dim3(64 * WN * WM), lds, s, g);
 }
 
-// The tile of the split changes no bits. The time of its grid: that of one tile
-// on a CU, and less for each further one on the busiest CU, by what they leave
-// each other (us at K = 1024, in the table below; 32x32 goes in stages of 64 k).
-// us by its order, then the best of launch_tiles<false>, which is ahead by up to a
+// The tile of the split changes no bits. Its grid takes the time of one tile on
+// a CU and less for each further one on the busiest CU, which fills what the
+// first leaves idle (us at K = 1024 in the table below; 32x32 goes in stages of
+// 64 k). us by its order, then the best of launch_tiles<false>, which is ahead by up to a
 // tenth on the smallest grids only: 31 x 1024 x 1024 12.0 / 20 / 25 / 29, 11.4; 253 x
 // 1024 x 1024 13 / 21 / 26 / 30, 12; 253 x 768 x 3072 31 / 56 / 69 / 81, 30; 545 x
 // 3072 x 768 36 / 28 / 39 / 25, 33; 1370 x 768 x 768 27 / 27 / 22 / 25, 24; 1370 x

@@ -297,6 +297,26 @@ def test_gemm_f32_rows_alone(gpu, pkg, lib, n, k, half):
         assert torch.equal(out.view(torch.int32), whole[:rows].view(torch.int32)), rows
 
 
+@pytest.mark.parametrize("k,rows", [(4, 2 ** 29 + 33), (64, 2 ** 27 + 33)])
+def test_gemm_f32_many_rows(gpu, pkg, lib, k, rows):
+    """More row tiles than grid x holds (k = 4: 2^32 threads of 32-row tiles), small
+    whole numbers, exact."""
+    torch = gpu
+    _announce("gemm_f32 many rows", k, rows)
+    small = torch.randint(-8, 9, (rows, 4), dtype=torch.int8, device="cuda")
+    ad = torch.zeros((rows, k), device="cuda")
+    ad[:, k - 4:] = small
+    bd = torch.zeros((1, k), device="cuda")
+    bd[0, k - 4:] = torch.tensor([1.0, -2.0, 3.0, 5.0], device="cuda")
+    out = torch.full((rows,), 7.5, device="cuda")
+    args = pkg.GemmF32Args()
+    args.a, args.lda, args.b, args.ldb = ptr(ad), k, ptr(bd), k
+    args.m, args.n, args.k, args.epilogue, args.out = rows, 1, k, 1, ptr(out)
+    ok(lib, lib.dav2_hip_gemm_f32(C.byref(args), stream(torch)))
+    want = small[:, 0].short() - 2 * small[:, 1].short() + 3 * small[:, 2].short() + 5 * small[:, 3].short()
+    assert torch.equal(out, want.float())
+
+
 def test_gemm_f32_rejects(gpu, pkg, lib):
     torch = gpu
     a = empty(torch, (8, 8), torch.float32)
