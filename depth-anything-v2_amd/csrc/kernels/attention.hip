@@ -252,7 +252,7 @@ __global__ __launch_bounds__(256) void attention_values_kernel(const float* __re
 // features 16 (l / 16) .. of its query.
 //
 // Softmax online, in fp32: running maximum per query, the sums rescaled only
-// where a maximum grew, p = exp(s - max) / 2^s by expf; the division comes last.
+// where a maximum grew, p = exp(s - max) / 2^n by expf; the division comes last.
 // Bounded by the fp32 MFMA (157 TFLOP/s). ViT-B 686x518 (T = 1814, 12
 // heads, 10.1 GFLOP): 495 us as scores + softmax + values (365 of them the
 // values) -> 134 us (76 TFLOP/s); 1370 tokens, 16 heads 372 -> 103; 5477 tokens,
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void f
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = v4f{0.f, 0.f, 0.f, 0.f};
     float maximum = kLowest, sum = 0.0f;  // sum: this lane's keys only
-    // Weights are exp / 2^s, 2^s >= tokens: no sum of weighted values passes the
+    // Weights are exp / 2^n, 2^n >= tokens: no sum of weighted values passes the
     // largest value (T = 5477, 16 heads 1247 -> 1256 us; the same bits elsewhere).
     const float share = __uint_as_float((95u + __clz(tokens - 1u)) << 23);
     v4f p[2];
